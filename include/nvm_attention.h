@@ -48,11 +48,14 @@ enum nvm_kv_dtype { NVM_KV_F16 = 0, NVM_KV_BF16 = 1, NVM_KV_F32 = 2, NVM_KV_I8 =
  * query row i (of L) sees positions j <= i + context_len - L.  Rows with no
  * visible position are zero.  Sums are float32, like the reference.
  *
- * L = 1 with f16/bf16 pages and D of 64 or 128 runs the split-context decode
- * kernel (the query heads of a kv head share every page read); other shapes
- * run a one-wavefront-per-row kernel.  Each page tensor must be below 2 GiB.
+ * L = 1 with f16/bf16/int8 pages and D of 64 or 128 runs the split-context
+ * decode kernel (the query heads of a kv head share every page read); L > 1
+ * with f16/bf16 pages and those D runs a matrix-core kernel over the pages;
+ * other shapes run a one-wavefront-per-row kernel (so do int8 pages or a
+ * query not aligned to 16 bytes).  Each page tensor must be below 2 GiB.
  * Workspace: nvm_paged_attention_workspace_size (zero bytes when no split is
- * needed; workspace may then be NULL).
+ * needed; workspace may then be NULL).  Int8 pages are also accepted without
+ * a workspace: the context is then not split.
  */
 int nvm_paged_attention_workspace_size(int64_t N, int64_t L, int64_t D, int64_t max_pages,
                                        int64_t page_size, int kv_dtype, int num_kv_heads,

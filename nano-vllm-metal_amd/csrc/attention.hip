@@ -8,7 +8,7 @@
 // j <= i + context_len - L, then the probability-weighted sum of the values.
 // Pages are [P, num_kv_heads, page_size, D] (cache/paged.py).
 //
-// Decode kernel (L = 1, f16/bf16 pages, D = 64 or 128).  A block owns one
+// Decode kernel (L = 1, f16/bf16/int8 pages, D = 64 or 128).  A block owns one
 // (request, kv head, group of up to RP query heads, context split): the query
 // heads that share a kv head read each key and value row once (grouped-query
 // sharing; the reference reads them once per query head).  Its eight
@@ -32,8 +32,16 @@
 //   * The wavefronts' (max, sum, output) partials meet in LDS; with more
 //     than one split per row they go to the workspace and a second launch
 //     combines them.
-// Other shapes (L > 1, f32 or int8 pages, other head dims) run one wavefront
-// per query row over the context, with the reference's formula per element.
+//   * Int8 pages run on the bf16 matrix cores: a code has at most 8
+//     significant bits, so its bf16 value is exact.  A lane loads 16 codes at
+//     a time (keys: dims 64kk + 16G .. +15, two chunks of a score MFMA; the
+//     query operand is built in that order).  The position's key scale
+//     multiplies its float32 score and its value scale the probability before
+//     the split into three parts, so every product stays exact and both sums
+//     float32.
+// Other shapes (L > 1 on f32 or int8 pages, f32 decode, other head dims) run
+// one wavefront per query row over the context, with the reference's formula
+// per element.
 #include <math.h>
 
 #include <algorithm>
@@ -104,12 +112,37 @@ __device__ __forceinline__ void split3(const float (&x)[8], u32x4 &p0, u32x4 &p1
   }
 }
 
-template <int DT, int DH, int RP, int NW>
+// Four int8 codes (the bytes of w) as bf16 values, exactly: the unsigned byte
+// code + 128 converts to float32, less 128 its upper 16 bits are the bf16.
+__device__ __forceinline__ u32x2 codes_to_bf16(uint32_t w) {
+  w ^= 0x80808080u;
+  const float f0 = (float)(w & 0xFFu) - 128.f, f1 = (float)((w >> 8) & 0xFFu) - 128.f;
+  const float f2 = (float)((w >> 16) & 0xFFu) - 128.f, f3 = (float)(w >> 24) - 128.f;
+  return u32x2{perm_b32(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u),
+               perm_b32(__float_as_uint(f3), __float_as_uint(f2), 0x07060302u)};
+}
+// Eight of a lane's sixteen codes (half 0 or 1) as an MFMA operand.
+__device__ __forceinline__ u32x4 codes8_to_bf16(u32x4 w, int half) {
+  const u32x2 a = codes_to_bf16(w[2 * half]), b = codes_to_bf16(w[2 * half + 1]);
+  return u32x4{a.x, a.y, b.x, b.y};
+}
+
+// I8: int8 pages with per-position scales (DT is then bf16).
+//
+// Int8 pages, one launch of (kv heads x splits) blocks instead of one
+// wavefront per query row that walks the context position by position (a
+// dependent load and a six-step lane reduction each): 8 requests of up to
+// 3000 positions at 32/4 heads of 128 took 3322 us a call that way (rows read
+// once per query head), KERNEL_US here.
+template <int DT, bool I8, int DH, int RP, int NW>
 __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(PagedArgs a) {
   using A = Act<DT>;
+  constexpr int ES = I8 ? 1 : 2;     // bytes per page element
+  constexpr int EL = 16 / ES;        // elements per 16-byte load
   constexpr int NC = DH / 32;        // 32-dim chunks of a score MFMA
   constexpr int NT = DH / 16;        // 16-dim output tiles of a P.V MFMA
-  constexpr int LPD = DH / 8;        // lanes per value row in the V loads, 8 dims each
+  constexpr int KL = DH / (4 * EL);  // 16-byte key loads per lane and position
+  constexpr int LPD = DH / EL;       // lanes per value row in the V loads, EL dims each
   constexpr int PG = 64 / LPD;       // position groups of the V loads
   constexpr int PPG = kTile / PG;    // positions per lane per tile
   constexpr int VP = DH + 8;         // LDS pitch of a staged value row (16-bit elements)
@@ -121,6 +154,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(PagedArgs a) {
   auto s_o = reinterpret_cast<float(*)[RP][DH]>(s_buf);
   __shared__ u32x4 s_q[NC][3][64];  // the score MFMAs' B operand, per lane
   __shared__ int s_row[NW][kTile];
+  __shared__ __attribute__((aligned(16))) float s_sc[I8 ? NW : 1][2][kTile];  // key, value scales
   __shared__ float s_m[NW][RP], s_l[NW][RP];
 
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -138,15 +172,15 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(PagedArgs a) {
   const int p0 = s * a.span;
   const int p1 = min(p0 + a.span, ctx);
 
-  // B operand of the score MFMAs (query head c16, dims 32k + 8G .. +7), the
-  // same for every wavefront: built once into LDS, read back per tile (it
+  // B operand of the score MFMAs (query head c16, dims 32k + 8G .. +7, or in
+  // the order of the 16-code key loads), the same for every wavefront: built once into LDS, read back per tile (it
   // would hold 12 * NC VGPRs for the whole loop)
   if (wv == 0) {
     const bool ok = c16 < nh;
     const float *qp = a.q + (n0 + (ok ? c16 : 0)) * DH;
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
-      const int d0 = 32 * k + 8 * G;
+      const int d0 = I8 ? 64 * (k >> 1) + 16 * G + 8 * (k & 1) : 32 * k + 8 * G;
       const f32x4 x0 = ok ? *(const f32x4 *)(qp + d0) : f32x4{0.f, 0.f, 0.f, 0.f};
       const f32x4 x1 = ok ? *(const f32x4 *)(qp + d0 + 4) : f32x4{0.f, 0.f, 0.f, 0.f};
       const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
@@ -159,10 +193,12 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(PagedArgs a) {
   }
   __syncthreads();
 
-  const uint32_t kv_bytes = (uint32_t)((int64_t)a.P * a.Hkv * a.page_size * DH * 2);
+  const uint32_t kv_bytes = (uint32_t)((int64_t)a.P * a.Hkv * a.page_size * DH * ES);
   const rsrc_t kr = make_rsrc(a.kp, kv_bytes), vr = make_rsrc(a.vp, kv_bytes);
+  const uint32_t sc_bytes = I8 ? kv_bytes / DH * 4 : 0;
+  const rsrc_t ksr = make_rsrc(a.ks, sc_bytes), vsr = make_rsrc(a.vs, sc_bytes);
   const int64_t bt_row = (int64_t)b * a.max_pages;
-  const int dd = 8 * (lane % LPD), pgrp = lane / LPD;
+  const int dd = EL * (lane % LPD), pgrp = lane / LPD;
 
   float m_run = -INFINITY, l_run = 0.f;  // head c16; l_run is this lane's share
   // O^T tiles: lane (c16, G) holds head c16, dims 16t + 4G + i
@@ -192,12 +228,13 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(PagedArgs a) {
                       : -1;
     }
     page_ids(t0 + NW * kTile, pg_next);
-    u32x4 kop[4][NC];
+    u32x4 kop[4][KL];
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int k = 0; k < NC; ++k)
-        kop[u][k] = bload16(kr, rowoff[u] >= 0 ? (rowoff[u] + 32 * k + 8 * G) * 2 : kMaskedOffset, 0);
+      for (int k = 0; k < KL; ++k)
+        kop[u][k] =
+            bload16(kr, rowoff[u] >= 0 ? (rowoff[u] + (4 * k + G) * EL) * ES : kMaskedOffset, 0);
     uint32_t vmask[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -205,13 +242,26 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(PagedArgs a) {
       if (G == 0) s_row[wv][16 * u + c16] = rowoff[u];
     }
     wave_lds_sync();
+    // the scales of position t0 + lane
+    float ksc = 0.f, vsc = 0.f;
+    if constexpr (I8) {
+      const int ro = s_row[wv][lane];
+      const int so = ro >= 0 ? ro / DH * 4 : kMaskedOffset;
+      ksc = __uint_as_float(bload4(ksr, so, 0));
+      vsc = __uint_as_float(bload4(vsr, so, 0));
+    }
     // the value rows, loaded with the keys (one memory round trip per tile):
-    // lane group pgrp holds dims dd..dd+7 of positions pgrp + PG*mm
+    // lane group pgrp holds dims dd..dd+EL-1 of positions pgrp + PG*mm
     u32x4 vv[PPG];
 #pragma unroll
     for (int mm = 0; mm < PPG; ++mm) {
       const int ro = s_row[wv][pgrp + PG * mm];
-      vv[mm] = bload16(vr, ro >= 0 ? (ro + dd) * 2 : kMaskedOffset, 0);
+      vv[mm] = bload16(vr, ro >= 0 ? (ro + dd) * ES : kMaskedOffset, 0);
+    }
+    if constexpr (I8) {
+      s_sc[wv][0][lane] = ksc;
+      s_sc[wv][1][lane] = vsc;
+      wave_lds_sync();
     }
 
     // S^T: lane (c16, G) holds head c16 at positions 16u + 4G + i
@@ -220,10 +270,16 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(PagedArgs a) {
     for (int u = 0; u < 4; ++u) {
       acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int k = 0; k < NC; ++k)
+      for (int k = 0; k < NC; ++k) {
+        u32x4 ka;
+        if constexpr (I8)
+          ka = codes8_to_bf16(kop[u][k >> 1], k & 1);
+        else
+          ka = kop[u][k];
 #pragma unroll
-        for (int part = 0; part < 3; ++part)
-          acc[u] = A::mfma16(kop[u][k], s_q[k][part][lane], acc[u]);
+        for (int part = 0; part < 3; ++part) acc[u] = A::mfma16(ka, s_q[k][part][lane], acc[u]);
+      }
+      if constexpr (I8) acc[u] *= *(const f32x4 *)&s_sc[wv][0][16 * u + 4 * G];
     }
     float sc[4][4];
     float tmax = -INFINITY;
@@ -264,8 +320,22 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(PagedArgs a) {
     for (int kc = 0; kc < 2; ++kc) {
 #pragma unroll
       for (int mm = kc * (32 / PG); mm < (kc + 1) * (32 / PG); ++mm)
-        *(u32x4 *)&s_v[wv][pgrp + PG * mm - 32 * kc][dd] = vv[mm];
+        if constexpr (I8) {
+          *(u32x4 *)&s_v[wv][pgrp + PG * mm - 32 * kc][dd] = codes8_to_bf16(vv[mm], 0);
+          *(u32x4 *)&s_v[wv][pgrp + PG * mm - 32 * kc][dd + 8] = codes8_to_bf16(vv[mm], 1);
+        } else {
+          *(u32x4 *)&s_v[wv][pgrp + PG * mm - 32 * kc][dd] = vv[mm];
+        }
       wave_lds_sync();
+      if constexpr (I8) {
+        // the value scales join the probabilities
+#pragma unroll
+        for (int u = 2 * kc; u < 2 * kc + 2; ++u) {
+          const f32x4 sv = *(const f32x4 *)&s_sc[wv][1][16 * u + 4 * G];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) pv[u][i] *= sv[i];
+        }
+      }
       const float x[8] = {pv[2 * kc][0], pv[2 * kc][1], pv[2 * kc][2], pv[2 * kc][3],
                           pv[2 * kc + 1][0], pv[2 * kc + 1][1], pv[2 * kc + 1][2],
                           pv[2 * kc + 1][3]};
@@ -459,7 +529,7 @@ struct AttnPlan {
 AttnPlan attn_plan(int64_t N, int64_t L, int64_t D, int64_t max_pages, int64_t page_size,
                    int kv_dtype, int Hkv, int Hq) {
   AttnPlan p{false, 0, 1, 1, 0};
-  p.decode = L == 1 && (kv_dtype == NVM_KV_F16 || kv_dtype == NVM_KV_BF16) && (D == 64 || D == 128);
+  p.decode = L == 1 && kv_dtype != NVM_KV_F32 && (D == 64 || D == 128);
   if (!p.decode) return p;
   const int R = Hq / Hkv;
   p.RP = R <= 8 ? 8 : 16;
@@ -480,22 +550,23 @@ size_t attn_workspace(const AttnPlan &p, int64_t N, int64_t D) {
   return o + (((size_t)N * p.S * 2 * sizeof(float) + 255) & ~(size_t)255);
 }
 
-template <int DT>
+template <int DT, bool I8>
 void launch_decode(const PagedArgs &a, int RP, int D, unsigned grid, hipStream_t st) {
+  const dim3 blk(64 * kDecodeWaves);
   if (D == 128) {
     if (RP == 8)
-      hipLaunchKernelGGL((paged_decode_kernel<DT, 128, 8, kDecodeWaves>), dim3(grid),
-                         dim3(64 * kDecodeWaves), 0, st, a);
+      hipLaunchKernelGGL((paged_decode_kernel<DT, I8, 128, 8, kDecodeWaves>), dim3(grid), blk, 0,
+                         st, a);
     else
-      hipLaunchKernelGGL((paged_decode_kernel<DT, 128, 16, kDecodeWaves>), dim3(grid),
-                         dim3(64 * kDecodeWaves), 0, st, a);
+      hipLaunchKernelGGL((paged_decode_kernel<DT, I8, 128, 16, kDecodeWaves>), dim3(grid), blk, 0,
+                         st, a);
   } else {
     if (RP == 8)
-      hipLaunchKernelGGL((paged_decode_kernel<DT, 64, 8, kDecodeWaves>), dim3(grid),
-                         dim3(64 * kDecodeWaves), 0, st, a);
+      hipLaunchKernelGGL((paged_decode_kernel<DT, I8, 64, 8, kDecodeWaves>), dim3(grid), blk, 0,
+                         st, a);
     else
-      hipLaunchKernelGGL((paged_decode_kernel<DT, 64, 16, kDecodeWaves>), dim3(grid),
-                         dim3(64 * kDecodeWaves), 0, st, a);
+      hipLaunchKernelGGL((paged_decode_kernel<DT, I8, 64, 16, kDecodeWaves>), dim3(grid), blk, 0,
+                         st, a);
   }
 }
 
@@ -571,8 +642,20 @@ int nvm_paged_attention(const float *q, int64_t N, int64_t L, int64_t D, const v
   ATTN_REQUIRE(kv_dtype != NVM_KV_I8 || P == 0 || (key_scales && value_scales),
                "paged_attention_int8: key_scales and value_scales are required");
 
-  const AttnPlan plan = attn_plan(N, L, D, max_pages, page_size, kv_dtype, num_kv_heads,
-                                  num_heads);
+  AttnPlan plan = attn_plan(N, L, D, max_pages, page_size, kv_dtype, num_kv_heads, num_heads);
+  if (plan.decode && kv_dtype == NVM_KV_I8) {
+    // the decode kernel's 16-byte loads of codes and queries need aligned
+    // tensors (the row kernel reads element by element), and a caller
+    // without a workspace gets one split per row
+    const uintptr_t align = (uintptr_t)q | (uintptr_t)key_pages | (uintptr_t)value_pages;
+    const int64_t cap = max_pages * page_size;
+    if ((align & 15) || cap > 0x7FFFFFFF - kDecodeWaves * kTile) {
+      plan = AttnPlan{false, 0, 1, 1, 0};
+    } else if (!workspace || workspace_bytes < attn_workspace(plan, N, D)) {
+      plan.S = 1;
+      plan.span = (int)cap;
+    }
+  }
   const size_t need = attn_workspace(plan, N, D);
   if (need && (!workspace || workspace_bytes < need))
     return set_error(NVM_ERR_WORKSPACE, "paged_attention: workspace of %zu bytes needed", need);
@@ -610,10 +693,12 @@ int nvm_paged_attention(const float *q, int64_t N, int64_t L, int64_t D, const v
     }
     const unsigned grid = (unsigned)(B * num_kv_heads * plan.HG * plan.S);
     if (grid == 0) return NVM_OK;
-    if (kv_dtype == NVM_KV_BF16)
-      launch_decode<DT_BF16>(a, plan.RP, (int)D, grid, st);
+    if (kv_dtype == NVM_KV_I8)
+      launch_decode<DT_BF16, true>(a, plan.RP, (int)D, grid, st);
+    else if (kv_dtype == NVM_KV_BF16)
+      launch_decode<DT_BF16, false>(a, plan.RP, (int)D, grid, st);
     else
-      launch_decode<DT_F16>(a, plan.RP, (int)D, grid, st);
+      launch_decode<DT_F16, false>(a, plan.RP, (int)D, grid, st);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(NVM_ERR_HIP, "paged_attention: %s", hipGetErrorString(e));
     if (plan.S > 1) {

@@ -178,6 +178,50 @@ def test_int8_multi_query_causal():
     _run(109, 2, 8, 4, 64, 16, [33, 100], L=4, causal=True, int8=True)
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,ps,lens", [
+    (8, 8, 64, 4, [1, 63, 64, 65, 0]),         # one head per kv head, edges of a 64-position tile
+    (10, 2, 128, 24, [511, 513, 700]),         # five per kv head, edges of a block's eight tiles
+    (24, 1, 128, 16, [129, 1030]),             # 24 per kv head: two groups of 16
+    (16, 1, 64, 128, [90]),                    # one request, pages of 128 slots
+    (32, 4, 128, 16, [2900, 17] + [1500] * 6),  # the serving heads over split contexts
+])
+def test_int8_decode_matrix_cores(Hq, Hkv, D, ps, lens):
+    """Int8 pages on the split decode kernel, with missing pages and page ids
+    past the pool."""
+    _run(140 + Hq, len(lens), Hq, Hkv, D, ps, lens, int8=True, holes=2, past_pool=1,
+         causal=Hq % 3 == 0)
+
+
+def test_int8_decode_without_workspace_or_alignment():
+    """Int8 decode calls accepted before the split kernel took them: no
+    workspace (one split per row), codes at an odd address (the row kernel).
+    Both agree with the split call within the sums' float32 rounding."""
+    from nano_vllm_metal_amd import _lib, paged_attention
+
+    g = torch.Generator(device=DEV).manual_seed(9)
+    B, Hq, Hkv, D, ps, mp = 2, 16, 4, 128, 16, 40
+    n = B * mp * Hkv * ps * D
+    q = torch.randn(B, Hq, 1, D, device=DEV, generator=g)
+    kc, vc = (torch.randint(-128, 128, (n + 1,), device=DEV, generator=g, dtype=torch.int8)
+              for _ in range(2))
+    ks, vs = (torch.rand(B * mp, Hkv, ps, 1, device=DEV, generator=g) * 0.02 for _ in range(2))
+    bt = torch.arange(B * mp, device=DEV, dtype=torch.int32).reshape(B, mp)
+    lens = torch.tensor([600, 333], device=DEV, dtype=torch.int32)
+    shape = (B * mp, Hkv, ps, D)
+    split = paged_attention(q, kc[:n].view(shape), vc[:n].view(shape), bt, lens, ps, ks, vs)
+    odd_k, odd_v = kc.clone(), vc.clone()
+    odd_k[1:], odd_v[1:] = kc[:n], vc[:n]
+    rows = paged_attention(q, odd_k[1:].view(shape), odd_v[1:].view(shape), bt, lens, ps, ks, vs)
+    out = torch.empty(B * Hq, 1, D, device=DEV)
+    _lib.check(_lib.load().nvm_paged_attention(
+        q.data_ptr(), B * Hq, 1, D, kc.data_ptr(), vc.data_ptr(), B * mp, ps, 3, ks.data_ptr(),
+        vs.data_ptr(), bt.data_ptr(), B, mp, lens.data_ptr(), D ** -0.5, 0, Hkv, Hq, 2,
+        out.data_ptr(), None, 0, _lib.stream_of(q.device)))
+    torch.cuda.synchronize()
+    torch.testing.assert_close(rows, split, rtol=RTOL, atol=ATOL)
+    torch.testing.assert_close(out.view_as(split), split, rtol=RTOL, atol=ATOL)
+
+
 @pytest.mark.parametrize("D", [96, 256, 32])
 def test_other_head_dims(D):
     _run(110, 2, 8, 2, D, 16, [77, 300])
