@@ -73,6 +73,21 @@ int nvm_moe_forward_residual_norm(const void *x, int64_t T, int64_t H, int64_t I
                                   size_t workspace_bytes, nvm_stream_t stream);
 
 /*
+ * Gate and up products of the dense MLP with SwiGLU: out = rnd(silu(rnd(a .
+ * gate^T)) * rnd(a . up^T)), silu's ops each rounded to the activation dtype.
+ * Replaces `silu(gate_proj(x)) * up_proj(x)` of `Qwen3MLP`
+ * (models/qwen3.py:176-184, layers/activation.py:21-24).  a [M, N] act; gate
+ * and up [K, N/8] words with scales and biases [K, N/group]; out [M, K] act.
+ * Shapes nvm_quantized_matmul runs on its exact float64 path (K <= 512 with
+ * M <= 64, N above 8192 or not a multiple of 64, K not a multiple of 16) are
+ * NVM_ERR_UNSUPPORTED.  Needs no workspace.
+ */
+int nvm_quantized_swiglu(const void *gate_scales, const void *gate_biases, const uint32_t *gate,
+                         const void *up_scales, const void *up_biases, const uint32_t *up,
+                         int group_size, int bits, const void *a, void *out, int64_t M, int64_t N,
+                         int64_t K, int dtype, nvm_stream_t stream);
+
+/*
  * Embedding lookup of a 4-bit affine-quantised table (MLX layout, as the
  * expert weights): out[t] = rnd(q * s + b) over row tokens[t], the value
  * computed in float32 and rounded once to the activation dtype.  Replaces

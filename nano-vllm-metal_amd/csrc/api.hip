@@ -400,6 +400,49 @@ const char *nvm_last_error(void) { return g_err.c_str(); }
 constexpr int64_t kExactOutMax = 512;
 constexpr int64_t kExactRowsMax = 64;
 
+// Kernel of a dense product of M rows over a reduction of N into K outputs.
+// The GEMV streams the weights once per 16- or 32-row chunk; the GEMM once,
+// but a block runs all N/64 k-steps in sequence, so a grid of fewer blocks
+// than CUs leaves the GEMM latency-bound.  The few-row kernel wherever it
+// applies; else the unit-list GEMV up to two chunks, and up to 32 chunks
+// while the GEMM grid would not fill the chip.
+static bool dense_decode(int64_t M, int64_t N, int64_t K) {
+  if (nvm::gemv_dense_supports(M, (int)N, (int)K)) return true;
+  const int64_t gemm_blocks = (M + nvm::kGemmBM - 1) / nvm::kGemmBM * ((K + 255) / 256);
+  return nvm::gemv_supports((int)N) &&
+         (M <= 32 || (M <= 512 && gemm_blocks < nvm::cu_count()));
+}
+
+static nvm::GroupedArgs dense_args(const void *scales, const void *biases, int group_size,
+                                   const void *a, const uint32_t *b, void *out, int64_t M,
+                                   int64_t N, int64_t K) {
+  nvm::GroupedArgs g{};
+  g.act = (const uint16_t *)a;
+  g.act_ld = N;
+  g.act_rows = M;
+  g.a_map = nullptr;
+  g.a_div = 1;
+  g.offsets = nullptr;  // one expert over all M rows
+  g.w0 = b;
+  g.s0 = (const uint16_t *)scales;
+  g.b0 = (const uint16_t *)biases;
+  g.R = (int)K;
+  g.K = (int)N;
+  g.gs = group_size;
+  g.E = 1;
+  g.out = (uint16_t *)out;
+  g.o_map = nullptr;
+  g.out_ld = K;
+  return g;
+}
+
+// Dense products that run on the expert products: everything but the
+// router-sized ones (which keep their exact sums) and odd shapes.
+static bool dense_on_products(int64_t M, int64_t N, int64_t K) {
+  return (K > kExactOutMax || M > kExactRowsMax) && K % 16 == 0 && N % 64 == 0 &&
+         N <= kMaxProductK;
+}
+
 int nvm_quantized_matmul(const void *scales, const void *biases, int group_size, int bits,
                          const void *a, const uint32_t *b, int transpose_b, void *out, int64_t M,
                          int64_t N, int64_t K, int dtype, nvm_stream_t stream) {
@@ -417,36 +460,38 @@ int nvm_quantized_matmul(const void *scales, const void *biases, int group_size,
   NVM_SUPPORTED(K * (N / 2) <= k2GiB && M * N * 2 <= k2GiB,
                 "quantized_matmul: operands of more than 2 GiB (a %lld bytes, b %lld bytes); "
                 "split the product", (long long)(M * N * 2), (long long)(K * (N / 2)));
-  if ((K > kExactOutMax || M > kExactRowsMax) && K % 16 == 0 && N % 64 == 0 && N <= kMaxProductK) {
-    nvm::GroupedArgs g{};
-    g.act = (const uint16_t *)a;
-    g.act_ld = N;
-    g.act_rows = M;
-    g.a_map = nullptr;
-    g.a_div = 1;
-    g.offsets = nullptr;  // one expert over all M rows
-    g.w0 = b;
-    g.s0 = (const uint16_t *)scales;
-    g.b0 = (const uint16_t *)biases;
-    g.R = (int)K;
-    g.K = (int)N;
-    g.gs = group_size;
-    g.E = 1;
-    g.out = (uint16_t *)out;
-    g.o_map = nullptr;
-    g.out_ld = K;
-    // The GEMV streams the weights once per 16-row chunk; the GEMM once, but
-    // a block runs all N/64 k-steps in sequence, so a grid of fewer blocks
-    // than CUs leaves the GEMM latency-bound.  GEMV up to two chunks, and up
-    // to 32 chunks while the GEMM grid would not fill the chip.
-    const int64_t gemm_blocks = (M + nvm::kGemmBM - 1) / nvm::kGemmBM * ((K + 255) / 256);
-    const bool decode = nvm::gemv_supports((int)N) &&
-                        (M <= 32 || (M <= 512 && gemm_blocks < nvm::cu_count()));
-    return run_products(dtype, decode, false, g, M, (hipStream_t)stream);
+  if (dense_on_products(M, N, K)) {
+    nvm::GroupedArgs g = dense_args(scales, biases, group_size, a, b, out, M, N, K);
+    return run_products(dtype, dense_decode(M, N, K), false, g, M, (hipStream_t)stream);
   }
   NVM_TRY_HIP(nvm::launch_route_partial(dtype, a, M, N, b, scales, biases, K, group_size, true,
                                         nullptr, out, nullptr, (hipStream_t)stream));
   return NVM_OK;
+}
+
+int nvm_quantized_swiglu(const void *gate_scales, const void *gate_biases, const uint32_t *gate,
+                         const void *up_scales, const void *up_biases, const uint32_t *up,
+                         int group_size, int bits, const void *a, void *out, int64_t M, int64_t N,
+                         int64_t K, int dtype, nvm_stream_t stream) {
+  if (int r = check_quant(group_size, bits, dtype)) return r;
+  NVM_REQUIRE(gate_scales && gate_biases && gate && up_scales && up_biases && up && a && out,
+              "quantized_swiglu: null pointer");
+  NVM_REQUIRE(M >= 0 && N > 0 && K > 0, "quantized_swiglu: bad shape M=%lld N=%lld K=%lld",
+              (long long)M, (long long)N, (long long)K);
+  NVM_REQUIRE(N % group_size == 0, "quantized_swiglu: N=%lld not divisible by group_size %d",
+              (long long)N, group_size);
+  if (M == 0) return NVM_OK;
+  NVM_SUPPORTED(K * (N / 2) <= k2GiB && M * N * 2 <= k2GiB,
+                "quantized_swiglu: operands of more than 2 GiB (a %lld bytes, weights %lld bytes); "
+                "split the product", (long long)(M * N * 2), (long long)(K * (N / 2)));
+  NVM_SUPPORTED(dense_on_products(M, N, K),
+                "quantized_swiglu: M=%lld N=%lld K=%lld takes two separate products",
+                (long long)M, (long long)N, (long long)K);
+  nvm::GroupedArgs g = dense_args(gate_scales, gate_biases, group_size, a, gate, out, M, N, K);
+  g.w1 = up;
+  g.s1 = (const uint16_t *)up_scales;
+  g.b1 = (const uint16_t *)up_biases;
+  return run_products(dtype, dense_decode(M, N, K), true, g, M, (hipStream_t)stream);
 }
 
 int nvm_route_workspace_size(int64_t T, int64_t H, int64_t E, size_t *bytes) {

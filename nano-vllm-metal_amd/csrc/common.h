@@ -175,6 +175,20 @@ __device__ __forceinline__ uint32_t perm_b32(uint32_t hi, uint32_t lo, uint32_t 
   return __builtin_amdgcn_perm(hi, lo, sel);
 }
 
+// Words (w0, w1, w2, w3) of a 16-byte load in lane group G hold codes
+// 32G + 8j.. of a 128-code group pair.  Exchanging the lower half-wave's
+// words 2-3 with the upper half-wave's words 0-1 leaves every lane with words
+// 0-1 from the first group and words 2-3 from the second: lane group G then
+// holds codes 32(G%2) + 16(G/2) + {0, 8} (first group) and 64 + the same
+// (second group).
+__device__ __forceinline__ u32x4 swap_pairs(u32x4 w) {
+  // v_permlane32_swap: lanes 32-63 of the first operand trade places with
+  // lanes 0-31 of the second
+  const auto a = __builtin_amdgcn_permlane32_swap(w.x, w.z, false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(w.y, w.w, false, false);
+  return u32x4{a[0], b[0], a[1], b[1]};
+}
+
 // Reorder 8 consecutive 16-bit values x0..x7 (held as 4 dwords) into the pair
 // order (x0,x4)(x1,x5)(x2,x6)(x3,x7) that nibble_pairs() produces for codes.
 __device__ __forceinline__ u32x4 pair_order(u32x4 d) {

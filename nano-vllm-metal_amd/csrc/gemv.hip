@@ -106,20 +106,6 @@ __device__ __forceinline__ uint32_t sb_at_tree(const u32x4 &v, int idx) {
   return (idx & 1) ? (d >> 16) : (d & 0xFFFFu);
 }
 
-// Words (w0, w1, w2, w3) of a 16-byte load in lane group G hold codes
-// 32G + 8j.. of a 128-code group pair.  Exchanging the lower half-wave's
-// words 2-3 with the upper half-wave's words 0-1 leaves every lane with words
-// 0-1 from the first group and words 2-3 from the second: lane group G then
-// holds codes 32(G%2) + 16(G/2) + {0, 8} (first group) and 64 + the same
-// (second group).
-__device__ __forceinline__ u32x4 swap_pairs(u32x4 w) {
-  // v_permlane32_swap: lanes 32-63 of the first operand trade places with
-  // lanes 0-31 of the second
-  const auto a = __builtin_amdgcn_permlane32_swap(w.x, w.z, false, false);
-  const auto b = __builtin_amdgcn_permlane32_swap(w.y, w.w, false, false);
-  return u32x4{a[0], b[0], a[1], b[1]};
-}
-
 template <bool DUAL, int GPW>
 struct GemvCfg {
   static constexpr int NM = DUAL ? 2 : 1;  // weight matrices per unit
@@ -636,6 +622,9 @@ hipError_t launch_gemv(int dtype, bool dual, const GroupedArgs &a, hipStream_t s
   // kernel's split of the reduction over a block's wavefronts keeps more
   // loads in flight: q_proj (2048 -> 4096) at one row takes 5.7 us here and
   // 9.4 us on gemv3.
+  // Dense products of few rows have a kernel of their own.
+  if (!a.offsets && a.E == 1 && !a.a_map && !a.o_map && gemv_dense_supports(a.act_rows, a.K, a.R))
+    return launch_gemv_dense(dtype, dual, a, st);
   GemvShape s;
   const bool old_ok = gemv_shape(a.K, a.R, s);
   if (gemv3_supports(a.K, a.R, a.E, a.gs)) {

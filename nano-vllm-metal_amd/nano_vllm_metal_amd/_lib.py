@@ -37,6 +37,7 @@ _SZ = ctypes.c_size_t
 # name -> argtypes; every function returns int status except the two getters
 SIGNATURES = {
     "nvm_quantized_matmul": [_P, _P, _I, _I, _P, _P, _I, _P, _I64, _I64, _I64, _I, _P],
+    "nvm_quantized_swiglu": [_P, _P, _P, _P, _P, _P, _I, _I, _P, _P, _I64, _I64, _I64, _I, _P],
     "nvm_route_workspace_size": [_I64, _I64, _I64, ctypes.POINTER(_SZ)],
     "nvm_moe_route": [_P, _I64, _I64, _P, _P, _P, _I64, _I, _I, _I, _I, _I, _P, _P, _P, _P, _SZ, _P],
     "nvm_dispatch_workspace_size": [_I64, _I64, ctypes.POINTER(_SZ)],

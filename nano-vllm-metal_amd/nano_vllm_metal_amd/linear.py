@@ -146,6 +146,45 @@ def quantized_matmul(scales: torch.Tensor, biases: torch.Tensor, group_size: int
     return out.reshape(*lead, K)
 
 
+def swiglu_supports(x: torch.Tensor, w_gate: QuantizedWeights, w_up: QuantizedWeights) -> bool:
+    """Whether ``quantized_swiglu`` takes these operands: one shape, group
+    size and dtype for both weights, and a product that ``quantized_matmul``
+    does not run on its exact float64 path."""
+    K, words = w_gate.weight.shape if w_gate.weight.dim() == 2 else (0, 0)
+    N = x.shape[-1]
+    M = x.numel() // N if N else 0
+    return (w_up.weight.shape == w_gate.weight.shape and words * 8 == N
+            and w_gate.group_size == w_up.group_size and w_gate.bits == w_up.bits == 4
+            and all(t.dtype == x.dtype and t.shape == (K, N // w_gate.group_size)
+                    for w in (w_gate, w_up) for t in (w.scales, w.biases))
+            and w_gate.group_size in (64, 128) and x.dtype in _lib.DTYPE_CODES
+            and M > 0 and (K > 512 or M > 64) and K % 16 == 0 and N % w_gate.group_size == 0
+            and N <= 8192)
+
+
+def quantized_swiglu(x: torch.Tensor, w_gate: QuantizedWeights, w_up: QuantizedWeights
+                     ) -> torch.Tensor:
+    """``silu(x . gate^T) * (x . up^T)`` in one launch, each op rounded to
+    ``x.dtype`` as the separate products and ``silu`` round it
+    (models/qwen3.py:176-184); operands as ``swiglu_supports``."""
+    lib = _lib.load()
+    if not swiglu_supports(x, w_gate, w_up):
+        raise ValueError("quantized_swiglu: operands take two separate products")
+    dev = _lib.require_device(x, w_gate.weight, w_gate.scales, w_gate.biases, w_up.weight,
+                              w_up.scales, w_up.biases)
+    *lead, N = x.shape
+    a = x.reshape(-1, N).contiguous()
+    gw, uw = (_u32_view_as_i32(w.weight).contiguous() for w in (w_gate, w_up))
+    gsc, gbi, usc, ubi = (t.contiguous() for w in (w_gate, w_up) for t in (w.scales, w.biases))
+    K = gw.shape[0]
+    out = torch.empty((a.shape[0], K), dtype=x.dtype, device=dev)
+    _lib.check(lib.nvm_quantized_swiglu(
+        gsc.data_ptr(), gbi.data_ptr(), gw.data_ptr(), usc.data_ptr(), ubi.data_ptr(),
+        uw.data_ptr(), w_gate.group_size, w_gate.bits, a.data_ptr(), out.data_ptr(), a.shape[0],
+        N, K, _lib.dtype_code(x.dtype), _lib.stream_of(dev)))
+    return out.reshape(*lead, K)
+
+
 def quantized_linear(x: torch.Tensor, w: QuantizedWeights,
                      bias: torch.Tensor | None = None) -> torch.Tensor:
     """``x . dequant(w)^T (+ bias)`` (linear.py:92-126) through the HIP matmul."""

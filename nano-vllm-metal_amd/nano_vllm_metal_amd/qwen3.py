@@ -34,7 +34,8 @@ import torch
 from .attention import causal_attention, causal_attention_supports, paged_attention
 from .fused import embedding, moe_residual_rms_norm, qk_norm_rope_store, residual_rms_norm
 from .kv_cache import PagedKVCache
-from .linear import QuantizedWeights, quantized_linear
+from .linear import (QuantizedWeights, quantized_linear, quantized_swiglu,
+                     swiglu_supports)
 from .moe import Moe
 
 
@@ -95,9 +96,11 @@ class DenseMLP:
         self.w_gate, self.w_up, self.w_down = w_gate, w_up, w_down
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
-        g = quantized_linear(x, self.w_gate)
-        u = quantized_linear(x, self.w_up)
-        return quantized_linear(silu(g) * u, self.w_down)
+        if swiglu_supports(x, self.w_gate, self.w_up):
+            h = quantized_swiglu(x, self.w_gate, self.w_up)
+        else:
+            h = silu(quantized_linear(x, self.w_gate)) * quantized_linear(x, self.w_up)
+        return quantized_linear(h, self.w_down)
 
 
 def silu(x: torch.Tensor) -> torch.Tensor:

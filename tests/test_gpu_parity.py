@@ -220,6 +220,57 @@ def test_quantized_matmul_dense_products(M, N, K, act, gs, path):
 
 
 @pytest.mark.parametrize("act", ["float16", "bfloat16"])
+@pytest.mark.parametrize("M,N,K,gs", [
+    (1, 128, 528, 128),     # one pair of groups: seven idle wavefronts, an odd number of row tiles
+    (15, 384, 1040, 64),    # three pairs over eight wavefronts
+    (16, 2048, 1024, 64),
+    (17, 4096, 1024, 128),  # sixteen wavefronts, a second chunk of one row
+    (33, 5120, 528, 64),    # reductions the unit-list GEMV does not hold
+    (48, 6144, 1024, 128),
+    (3, 8192, 528, 64),     # more pairs a wavefront than its ring holds
+])
+def test_few_row_dense_products(M, N, K, act, gs):
+    """The few-row kernel against the exactly rounded results: its sums are
+    float32 over exact products, so an output differs only where the exact
+    value lies within the sums' rounding (far below an act ulp) of a tie."""
+    from nano_vllm_metal_amd import quantized_matmul
+
+    rng = np.random.default_rng(M + N + K)
+    a = O.round_act(rng.standard_normal((M, N)), act)
+    w = O.round_act(rng.standard_normal((K, N)) * 0.02, act)
+    wq, s, b = O.quantize(w, gs, 4, act)
+    out = quantized_matmul(to_act(s, act, DEV), to_act(b, act, DEV), gs, 4, to_act(a, act, DEV),
+                           to_words(wq, DEV), transpose_b=True)
+    ref = O.quantized_matmul(a, wq, s, b, gs, act)
+    assert_moe_close(out, ref, act, f"few rows {M}x{N}x{K}", mae_rel=True)
+    assert np.mean(to_np(out) == ref) > 0.97
+
+
+@pytest.mark.parametrize("act", ["float16", "bfloat16"])
+@pytest.mark.parametrize("M,gs", [(1, 64), (16, 128), (33, 64), (700, 64)])
+def test_swiglu_product_matches_separate_products(M, gs, act):
+    """quantized_swiglu (few-row, unit-list GEMV and GEMM) against silu and
+    multiply on the two separate products, each op rounded to act: bit
+    identical where both run the same kernel's sums, and in all cases within
+    the block tolerance."""
+    from nano_vllm_metal_amd.linear import quantized_linear, quantized_swiglu
+    from nano_vllm_metal_amd.qwen3 import silu
+
+    rng = np.random.default_rng(M)
+    N, K = 2048, 6144
+    ws = []
+    for _ in range(2):
+        w = O.round_act(rng.standard_normal((K, N)) * 0.02, act)
+        ws.append(qweights(O.quantize(w, gs, 4, act), act, gs, DEV))
+    x = to_act(O.round_act(rng.standard_normal((M, N)), act), act, DEV)
+    h = quantized_swiglu(x, *ws)
+    ref = silu(quantized_linear(x, ws[0])) * quantized_linear(x, ws[1])
+    assert_moe_close(h, to_np(ref), act, f"swiglu M={M}", mae_rel=True)
+    if M in (1, 16):
+        assert torch.equal(h, ref)
+
+
+@pytest.mark.parametrize("act", ["float16", "bfloat16"])
 @pytest.mark.parametrize("gs", [64, 128])
 def test_torch_quantizer_on_gpu(act, gs):
     """The MLX affine quantizer that builds every benchmark and test weight set,
