@@ -172,8 +172,16 @@ int run_route_dispatch(int dtype, const void *x, int64_t T, int64_t H, const uin
     // this path does not use (T * E doubles at least)
     int32_t *hist = (int32_t *)partial;
     void *xo = dtype == NVM_DTYPE_BF16 ? xh : nullptr;
-    NVM_TRY_HIP(nvm::launch_route_i8_fin(dtype, x, T, H, wr, sr, br, E, gs, k, norm, ids, scores,
-                                         hist, xo, xo ? xsh : nullptr, st));
+    if (const int splits = nvm::route_i8_split(T, H, E)) {
+      hist = (int32_t *)(partial + (size_t)splits * T * E);
+      NVM_TRY_HIP(nvm::launch_route_i8(dtype, x, T, H, wr, sr, br, E, gs, partial, nullptr, st,
+                                       splits, xo, xo ? xsh : nullptr));
+      NVM_TRY_HIP(nvm::launch_route_fin_hist(dtype, partial, splits, T, E, k, norm, ids, scores,
+                                             hist, st));
+    } else {
+      NVM_TRY_HIP(nvm::launch_route_i8_fin(dtype, x, T, H, wr, sr, br, E, gs, k, norm, ids, scores,
+                                           hist, xo, xo ? xsh : nullptr, st));
+    }
     NVM_TRY_HIP(nvm::launch_dispatch_hist(ids, T * k, E, hist, (T + 15) / 16, 16 * k, offsets,
                                           sorted, st));
     if (xh_done) *xh_done = xo != nullptr;

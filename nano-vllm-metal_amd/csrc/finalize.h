@@ -196,17 +196,28 @@ __device__ __forceinline__ void finalize_token64(const double *__restrict__ part
       sum[jj] = (0.0 + __builtin_bit_cast(double, u32x2{v[jj].x, v[jj].y})) +
                 __builtin_bit_cast(double, u32x2{v[jj].z, v[jj].w});
   } else {
+    // eight splits' loads in flight at a time, added in split order
     after_loads();
     sum[0] = sum[1] = 0.0;
-    for (int z = 0; z < splits; ++z) {
-      u32x2 v[2];
+    for (int z0 = 0; z0 < splits; z0 += 8) {
+      u32x4 v[2][4];
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) {
         const int e = c + 16 * (2 * G + jj);
-        v[jj] = bload8(pr, tok && e < E ? ((t * E + e) * splits + z) * 8 : kMaskedOffset, 0);
+        const int off = tok && e < E ? ((t * E + e) * splits + z0) * 8 : kMaskedOffset;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          v[jj][q] = bload16(pr, z0 + 2 * q < splits ? off + 16 * q : kMaskedOffset, 0);
       }
 #pragma unroll
-      for (int jj = 0; jj < 2; ++jj) sum[jj] += __builtin_bit_cast(double, v[jj]);
+      for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          sum[jj] += __builtin_bit_cast(double, u32x2{v[jj][q].x, v[jj][q].y});
+          // (an odd count leaves the last pair's second value to the next row)
+          if (z0 + 2 * q + 1 < splits)
+            sum[jj] += __builtin_bit_cast(double, u32x2{v[jj][q].z, v[jj][q].w});
+        }
     }
   }
   double lg[2], p[2];

@@ -111,7 +111,8 @@ bool route_i8_applies(int64_t T, int64_t H);
 int route_i8_splits(int64_t T, int64_t H, int64_t E);
 hipError_t launch_route_i8(int dtype, const void *x, int64_t T, int64_t H, const uint32_t *wr,
                            const void *sr, const void *br, int64_t E, int gs, double *partial,
-                           unsigned *done, hipStream_t st);
+                           unsigned *done, hipStream_t st, int splits = 0, void *xh = nullptr,
+                           uint8_t *xsh = nullptr);
 // The whole routing of batches the int8 router takes, for E <= 128 and
 // top-k <= 16 (and at most 64 groups a row): logits, softmax, top-k and
 // renormalisation in one launch of one block per 16 tokens, which writes
@@ -124,6 +125,15 @@ hipError_t launch_route_i8_fin(int dtype, const void *x, int64_t T, int64_t H, c
                                const void *sr, const void *br, int64_t E, int gs, int k, int norm,
                                int32_t *ids, void *scores, int32_t *counts, void *xh,
                                uint8_t *xsh, hipStream_t st);
+// The same routing in two launches for batches whose T / 16 blocks leave the
+// chip idle: launch_route_i8's partial logits (with xh/xsh as above) over
+// route_i8_split hidden splits (0: the one launch is taken), then
+// launch_route_fin_hist.  The splits leave room for its histograms behind the
+// partials in a workspace of route_workspace_splits partials.
+int route_i8_split(int64_t T, int64_t H, int64_t E);
+hipError_t launch_route_fin_hist(int dtype, const double *partial, int splits, int64_t T,
+                                 int64_t E, int k, int norm, int32_t *ids, void *scores,
+                                 int32_t *counts, hipStream_t st);
 // `done` (may be NULL) is a counter the partial launch zeroes for the fused
 // finalise-and-dispatch launch that follows it.
 hipError_t launch_route_partial(int dtype, const void *x, int64_t T, int64_t H, const uint32_t *wr,

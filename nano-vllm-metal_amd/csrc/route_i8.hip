@@ -279,8 +279,9 @@ template <int DT>
 __global__ __launch_bounds__(64 * kI8Waves, 2) void route_i8_kernel(
     const uint16_t *__restrict__ x, int T, int H, const uint32_t *__restrict__ wr,
     const uint16_t *__restrict__ sr, const uint16_t *__restrict__ br, int E, int gs, int n_tt,
-    int splits, double *__restrict__ part, unsigned *__restrict__ done) {
-  hoist_args(x, T, H, wr, sr, br, E, gs, n_tt, splits, part, done);
+    int splits, double *__restrict__ part, unsigned *__restrict__ done,
+    uint16_t *__restrict__ xh, uint8_t *__restrict__ xsh) {
+  hoist_args(x, T, H, wr, sr, br, E, gs, n_tt, splits, part, done, xh, xsh);
   extern __shared__ double s_red[];  // [kI8Waves - 1][tile][row][lane], then the staged s/b
   // the finalising launch that follows counts its blocks from zero
   if (done && blockIdx.x == 0 && threadIdx.x == 0) *done = 0u;
@@ -310,8 +311,9 @@ __global__ __launch_bounds__(64 * kI8Waves, 2) void route_i8_kernel(
   i8_stage_sb(srr, brr, e0, GPR, g0, g1, s_sb, threadIdx.x, 64 * kI8Waves);
   __syncthreads();
   double acc[kI8Tiles][4];
-  i8_wave_sums<DT>(xr, wrr, xo, e0, HW, gs, GPR, g0, k0, k1, s_sb, acc, nullptr, false,
-                   nullptr);
+  // (the first expert range's blocks write the fp16 copy)
+  i8_wave_sums<DT>(xr, wrr, xo, e0, HW, gs, GPR, g0, k0, k1, s_sb, acc, ec == 0 ? xh : nullptr,
+                   ta < T, xsh ? xsh + (int64_t)ta * KS : nullptr);
 
   // the wavefronts' partials meet in LDS, added in wavefront order
   // (a lane's slots are 512 bytes apart: compile-time offsets from one base)
@@ -336,6 +338,34 @@ __global__ __launch_bounds__(64 * kI8Waves, 2) void route_i8_kernel(
         if (t < T && e < E) part[((int64_t)t * E + e) * splits + z] = v;
       }
   }
+}
+
+// Finalise of 16 tokens a block, one a wavefront, from the partial logits
+// [T][E][splits] (added in split order): ids, scores and the block's expert
+// histogram, as route_i8_fin_kernel leaves them (finalize_token64 forms the
+// same bits).
+template <int DT>
+__global__ __launch_bounds__(1024) void route_fin_hist_kernel(
+    const double *__restrict__ part, int splits, int T, int E, int k, int norm,
+    int32_t *__restrict__ ids, uint16_t *__restrict__ scores, int32_t *__restrict__ counts) {
+  hoist_args(part, splits, T, E, k, norm, ids, scores, counts);
+  __shared__ int s_ids[16 * kRowTopK];
+  __shared__ uint16_t s_sc[16 * kRowTopK];
+  __shared__ uint64_t s_mask[kRowExperts];
+  const int tid = threadIdx.x, tt = blockIdx.x;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (tid < kRowExperts) s_mask[tid] = 0ull;
+  __syncthreads();
+  const int nt = min(16, T - tt * 16);
+  if (wv < nt)
+    finalize_token64<DT>(part + (int64_t)tt * 16 * E * splits, splits, wv, nt, E, k, norm, s_ids,
+                         s_sc, s_mask);
+  __syncthreads();
+  if (tid < nt * k) {
+    ids[(int64_t)tt * 16 * k + tid] = s_ids[tid];
+    scores[(int64_t)tt * 16 * k + tid] = s_sc[tid];
+  }
+  if (tid < E) counts[(int64_t)tt * E + tid] = __popcll(s_mask[tid]);
 }
 
 // The whole routing of 16 tokens in one block (E <= 128, k <= 16): 4 n_ec
@@ -466,6 +496,21 @@ bool route_i8_fin_supports(int64_t T, int64_t H, int64_t E, int gs, int k) {
          H / gs <= kSbGroups;
 }
 
+// The one-launch routing runs T / 16 blocks, each a chain of a quarter of the
+// hidden columns' k-steps and the finalise: 30 us at any T up to 4096 (H
+// 2048), 58 us at H 4096.  Over hidden splits the partial logits of 150
+// tokens take 8 us and the finalise 6.  The layer's time with one launch /
+// two (bf16): H 2048, 150 tokens 170.7 / 155.2 us, 512 183.8 / 169.9, 1000
+// 215.5 / 219.2, 2048 312.4 / 305.6, 3000 376.0 / 379.3; H 4096, 150 tokens
+// 484.5 / 451.5, 700 556.5 / 536.6, 1000 625.6 / 614.1.
+constexpr int64_t kRouteSplitTokens = 2048;
+int route_i8_split(int64_t T, int64_t H, int64_t E) {
+  if (T > kRouteSplitTokens) return 0;
+  const int s = route_i8_splits(T, H, E);
+  if (s < route_workspace_splits(T, H, E)) return s;
+  return s >= 2 && (H / 64 + s / 2 - 1) / (s / 2) + 1 <= kSbGroups ? s / 2 : 0;
+}
+
 hipError_t launch_route_i8_fin(int dtype, const void *x, int64_t T, int64_t H, const uint32_t *wr,
                                const void *sr, const void *br, int64_t E, int gs, int k, int norm,
                                int32_t *ids, void *scores, int32_t *counts, void *xh,
@@ -499,21 +544,36 @@ hipError_t launch_route_i8_fin(int dtype, const void *x, int64_t T, int64_t H, c
 
 hipError_t launch_route_i8(int dtype, const void *x, int64_t T, int64_t H, const uint32_t *wr,
                            const void *sr, const void *br, int64_t E, int gs, double *partial,
-                           unsigned *done, hipStream_t st) {
+                           unsigned *done, hipStream_t st, int splits, void *xh, uint8_t *xsh) {
+  if (xh && (dtype != DT_BF16 || !xsh)) return hipErrorInvalidValue;
   if (H % 64 != 0 || gs % 64 != 0 || T <= 0) return hipErrorInvalidValue;
   if ((H / 64 + kI8MaxSplits - 1) / kI8MaxSplits + 1 > kSbGroups) return hipErrorInvalidValue;
   const int n_tt = (int)((T + 15) / 16);
   const int n_ec = (int)((E + 16 * kI8Tiles - 1) / (16 * kI8Tiles));
-  const int splits = route_i8_splits(T, H, E);
+  if (splits <= 0) splits = route_i8_splits(T, H, E);
   const dim3 grid((unsigned)(n_tt * n_ec * splits)), block(64 * kI8Waves);
   if (dtype == DT_BF16)
     hipLaunchKernelGGL(route_i8_kernel<DT_BF16>, grid, block, kI8Lds, st, (const uint16_t *)x,
                        (int)T, (int)H, wr, (const uint16_t *)sr, (const uint16_t *)br, (int)E, gs,
-                       n_tt, splits, partial, done);
+                       n_tt, splits, partial, done, (uint16_t *)xh, xsh);
   else
     hipLaunchKernelGGL(route_i8_kernel<DT_F16>, grid, block, kI8Lds, st, (const uint16_t *)x,
                        (int)T, (int)H, wr, (const uint16_t *)sr, (const uint16_t *)br, (int)E, gs,
-                       n_tt, splits, partial, done);
+                       n_tt, splits, partial, done, nullptr, nullptr);
+  return hipGetLastError();
+}
+
+hipError_t launch_route_fin_hist(int dtype, const double *partial, int splits, int64_t T,
+                                 int64_t E, int k, int norm, int32_t *ids, void *scores,
+                                 int32_t *counts, hipStream_t st) {
+  if (T <= 0 || E > kRowExperts || k > kRowTopK) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)((T + 15) / 16));
+  if (dtype == DT_BF16)
+    hipLaunchKernelGGL(route_fin_hist_kernel<DT_BF16>, grid, dim3(1024), 0, st, partial, splits,
+                       (int)T, (int)E, k, norm, ids, (uint16_t *)scores, counts);
+  else
+    hipLaunchKernelGGL(route_fin_hist_kernel<DT_F16>, grid, dim3(1024), 0, st, partial, splits,
+                       (int)T, (int)E, k, norm, ids, (uint16_t *)scores, counts);
   return hipGetLastError();
 }
 

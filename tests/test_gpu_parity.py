@@ -220,6 +220,31 @@ def test_quantized_matmul_dense_products(M, N, K, act, gs, path):
 
 
 @pytest.mark.parametrize("act", ["float16", "bfloat16"])
+@pytest.mark.parametrize("T,H,E,k", [
+    (128, 2048, 128, 8),   # whole 16-token blocks, eight hidden splits
+    (129, 2048, 40, 3),    # a last block of one token
+    (333, 4096, 128, 8),   # half the splits (room for the histograms)
+    (2048, 1024, 64, 16),  # the largest batch, fewer splits
+    (2049, 1024, 64, 16),  # beyond it: one launch
+    (200, 192, 128, 8),    # one split only: one launch
+])
+def test_split_prefill_routing(T, H, E, k, act):
+    """Routing of mid-sized batches in two launches: ids, scores, offsets and
+    sorted pairs equal route_topk followed by moe_dispatch, bit for bit."""
+    from nano_vllm_metal_amd import moe_dispatch, route_and_dispatch, route_topk
+
+    rng = np.random.default_rng(T + H)
+    x = to_act(O.round_act(rng.standard_normal((T, H)), act), act, DEV)
+    w = qweights(O.quantize(O.round_act(rng.standard_normal((E, H)) * 0.05, act), 64, 4, act),
+                 act, 64, DEV)
+    ids, scores, offsets, pairs = route_and_dispatch(x, w, k, True)
+    _, ids2, scores2 = route_topk(x, w, k, True)
+    offsets2, pairs2 = moe_dispatch(ids2, E)
+    assert torch.equal(ids, ids2.view(torch.int32)) and torch.equal(scores, scores2)
+    assert torch.equal(offsets, offsets2) and torch.equal(pairs, pairs2)
+
+
+@pytest.mark.parametrize("act", ["float16", "bfloat16"])
 @pytest.mark.parametrize("M,N,K,gs", [
     (1, 128, 528, 128),     # one pair of groups: seven idle wavefronts, an odd number of row tiles
     (15, 384, 1040, 64),    # three pairs over eight wavefronts
