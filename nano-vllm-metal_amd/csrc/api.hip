@@ -230,6 +230,8 @@ int run_products(int dtype, bool decode, bool dual, nvm::GroupedArgs &g, int64_t
                 (long long)(g.act_rows * g.act_ld * 2));
   if (decode) {
     NVM_TRY_HIP(nvm::launch_gemv(dtype, dual, g, st));
+  } else if (const int blocks = nvm::gemm_mid_blocks(dual, g, pairs)) {
+    NVM_TRY_HIP(nvm::launch_gemm_mid(dtype, dual, blocks, g, pairs, st));
   } else {
     const int64_t max_tiles = pairs / nvm::kGemmBM + g.E;
     NVM_TRY_HIP(nvm::launch_gemm(dtype, dual, g, max_tiles, st));

@@ -45,6 +45,7 @@
 #include <stdlib.h>
 
 #include "common.h"
+#include "gemm_common.h"
 #include "internal.h"
 
 namespace nvm {
@@ -69,71 +70,6 @@ constexpr int W_WAVE = 32 * W_PITCH;
 // two activation stages (one k-step each), two weight stages (a k-step pair
 // each) and the four wavefronts' scale/bias windows: 77 KB, two blocks per CU
 constexpr int kGemmLds = 2 * A_STAGE + 2 * B_STAGE + 4 * W_WAVE;
-
-typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ uint32_t pk_fma_h(uint32_t a, uint32_t b, uint32_t c) {  // v_pk_fma_f16
-  return __builtin_bit_cast(uint32_t,
-                            __builtin_elementwise_fma(__builtin_bit_cast(h2_t, a),
-                                                      __builtin_bit_cast(h2_t, b),
-                                                      __builtin_bit_cast(h2_t, c)));
-}
-__device__ __forceinline__ uint32_t pk_add_h(uint32_t a, uint32_t b) {  // v_pk_add_f16
-  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2_t, a) + __builtin_bit_cast(h2_t, b));
-}
-
-// One packed word (codes q0..q7, q_i at bits 4i) -> the 8 weights q_i*s + b
-// as fp16, each the correctly rounded value of the exact q*s + b (one
-// v_pk_fma_f16 per pair, single rounding), in the pair order
-// (q0,q4)(q1,q5)(q2,q6)(q3,q7): the codes become the exact fp16 values
-// 1024 + q by OR-ing them into the mantissa of 1024.0 (whose ulp is 1) and
-// 1024 is then taken off exactly.  s2, b2: (s, s) and (b, b) as fp16 pairs.
-__device__ __forceinline__ u32x4 dequant8_h(uint32_t w, uint32_t s2, uint32_t b2, uint32_t mask,
-                                            uint32_t magic) {
-  u32x4 d = nibble_pairs_v<0>(w, mask, magic);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) d[i] = pk_fma_h(pk_add_h(d[i], 0xE400E400u), s2, b2);
-  return d;
-}
-
-// Eight consecutive activations x0..x7 (one 16-byte chunk of a row) -> fp16
-// in the pair order (x0,x4)(x1,x5)(x2,x6)(x3,x7) of dequant8_h.  (Activations
-// that arrive in fp16, GroupedArgs::act_h, are in that order already.)  bf16 values
-// convert exactly (fp16 carries more significand bits) within fp16's range;
-// v_cvt_pkrtz_f16_f32 only rounds below it (|x| < 2^-14, with a contribution
-// far under the product's rounding) and saturates above 65504.
-template <int DT>
-__device__ __forceinline__ u32x4 act_to_h(u32x4 v) {
-  if constexpr (DT == DT_F16) {
-    return pair_order(v);
-  } else {
-    u32x4 o;
-    const float x0 = __uint_as_float(v.x << 16), x1 = __uint_as_float(v.x & 0xFFFF0000u);
-    const float x2 = __uint_as_float(v.y << 16), x3 = __uint_as_float(v.y & 0xFFFF0000u);
-    const float x4 = __uint_as_float(v.z << 16), x5 = __uint_as_float(v.z & 0xFFFF0000u);
-    const float x6 = __uint_as_float(v.w << 16), x7 = __uint_as_float(v.w & 0xFFFF0000u);
-    o.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0, x4));
-    o.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x1, x5));
-    o.z = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x2, x6));
-    o.w = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x3, x7));
-    return o;
-  }
-}
-
-// A scale or bias (act bits) as fp16 bits; bf16 values convert with round to
-// nearest even (exactly, inside fp16's normal range).
-template <int DT>
-__device__ __forceinline__ uint32_t sb_h(uint32_t bits) {
-  if constexpr (DT == DT_F16)
-    return bits & 0xFFFFu;
-  else
-    return __builtin_bit_cast(uint16_t, (_Float16)__uint_as_float(bits << 16));
-}
-
-__device__ __forceinline__ f32x16 mfma32_h(u32x4 a, u32x4 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
-                                                __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
 
 // AH: the activations arrive already in fp16 (GroupedArgs::act_h).
 template <int DT, bool DUAL, bool AH>
@@ -379,9 +315,7 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(const GroupedArgs a, int n
     sc[1] = perm_b32(v.y, v.y, 0x01000100u);
     bi[1] = perm_b32(v.y, v.y, 0x03020302u);
   };
-  // nibble-expansion constants in registers (one v_and_or_b32 per dword)
-  const uint32_t nib_mask = sgpr_const(0x000F000Fu);
-  const uint32_t magic = vgpr_const(0x64006400u);  // fp16 (1024, 1024)
+  const DeqConst dk = deq_const();
   // Software-pipelined over the four 16-wide chunks: the A reads and the
   // dequantisation of chunk c + 1 are issued ahead of chunk c's MFMAs.
   // NA: the 32-row blocks of routed rows computed (the tile's rows lie in
@@ -402,7 +336,7 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(const GroupedArgs a, int n
     };
     auto deq = [&](int c, u32x4 (&bf)[2]) {
 #pragma unroll
-      for (int s = 0; s < 2; ++s) bf[s] = dequant8_h(bw[s][c], sc[s], bi[s], nib_mask, magic);
+      for (int s = 0; s < 2; ++s) bf[s] = dequant8_h(bw[s][c], sc[s], bi[s], dk);
     };
     u32x4 af[4], bf[2];
     load_a(0, af);
@@ -819,8 +753,7 @@ __global__ __launch_bounds__(256, 2) void gemm_dma_kernel(const GroupedArgs a, i
     sc[1] = perm_b32(v.y, v.y, 0x01000100u);
     bi[1] = perm_b32(v.y, v.y, 0x03020302u);
   };
-  const uint32_t nib_mask = sgpr_const(0x000F000Fu);
-  const uint32_t magic = vgpr_const(0x64006400u);
+  const DeqConst dk = deq_const();
   // this lane's A read offsets within a stage: row l32 (+ 32 i), chunk
   // 4 h + c at slot (4 h + c) ^ (l32 & 7) ^ ((l32 >> 3) & 1)
   int a_rd[4];
@@ -838,7 +771,7 @@ __global__ __launch_bounds__(256, 2) void gemm_dma_kernel(const GroupedArgs a, i
     };
     auto deq = [&](int c, u32x4 (&bf)[2]) {
 #pragma unroll
-      for (int s = 0; s < 2; ++s) bf[s] = dequant8_h(bw[s][c], sc[s], bi[s], nib_mask, magic);
+      for (int s = 0; s < 2; ++s) bf[s] = dequant8_h(bw[s][c], sc[s], bi[s], dk);
     };
     u32x4 af[4], bf[2];
     load_a(0, af);

@@ -248,12 +248,13 @@ hipError_t launch_t(bool dual, const GroupedArgs &a, hipStream_t st) {
 // 4096: 16 rows 7.7 / 10.7, 32 rows 13.1 / 12.7; up to 1.5 blocks a CU (the
 // longer ring leaves registers for fewer).  Where that GEMV does not hold
 // the reduction (K 5120, 6144, 8192) the alternative is the GEMM, whose few
-// blocks run every k-step in sequence: 6144 -> 2048 5 rows 8.6 / 77.1, 64
-// rows 16.4 / 79.9, 256 rows 58.1 / 98.3; up to 10 blocks a CU there.
+// blocks run every k-step in sequence (gemm_mid.hip): 6144 -> 2048 128 rows
+// 30.5 / 47, 160 rows 37.6 / 47, 200 rows 51.5 / 47; up to 5 blocks a CU
+// there.
 bool gemv_dense_supports(int64_t M, int K, int R) {
   if (M < 1 || M > 4096 || K % 128 || K > 8192 || R % 16) return false;
   const int64_t blocks = (M + 15) / 16 * (R / 16), cu = cu_count();
-  return 2 * blocks <= (K <= 2048 ? 5 : 3) * cu || (!gemv_supports(K) && blocks <= 10 * cu);
+  return 2 * blocks <= (K <= 2048 ? 5 : 3) * cu || (!gemv_supports(K) && blocks <= 5 * cu);
 }
 
 hipError_t launch_gemv_dense(int dtype, bool dual, const GroupedArgs &a, hipStream_t st) {

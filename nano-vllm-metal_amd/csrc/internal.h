@@ -195,6 +195,13 @@ constexpr int kGemmBM = 128;   // prefill tile rows (routed pairs)
 constexpr int kGemmBN = 128;   // prefill tile columns per weight matrix
 hipError_t launch_gemm(int dtype, bool dual, const GroupedArgs &a, int64_t max_m_tiles,
                        hipStream_t st);
+// The same products on m-tiles of one or two 32-row blocks with a deeper
+// weight stream (gemm_mid.hip), bit-identical, for mid-sized batches:
+// gemm_mid_blocks says how many 32-row blocks a tile should have (0: the
+// 128-row kernels are taken).
+int gemm_mid_blocks(bool dual, const GroupedArgs &a, int64_t pairs);
+hipError_t launch_gemm_mid(int dtype, bool dual, int blocks, const GroupedArgs &a, int64_t pairs,
+                           hipStream_t st);
 // bf16 x [n] -> its fp16 copy for the prefill GEMMs: each 64-value group
 // shifted (bf16_to_f16_pairs) with its shift in sh [n / 64], each 16-byte
 // chunk in the pair order of GroupedArgs::act_h; n a multiple of 64, `out`

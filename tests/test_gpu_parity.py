@@ -219,6 +219,57 @@ def test_quantized_matmul_dense_products(M, N, K, act, gs, path):
     assert same > 0.9, f"{path}: {same:.3f} of the outputs equal the rounded exact result"
 
 
+def _packed(rng, E, out, inn, gs, act):
+    """Random 4-bit expert weights: words, and scales and biases of N(0, 0.02) groups."""
+    words = rng.integers(0, 2**32, (E, out, inn // 8), dtype=np.uint64).astype(np.uint32)
+    s = O.round_act(rng.uniform(0.006, 0.01, (E, out, inn // gs)), act)
+    return words, s, O.round_act(-7.5 * s, act)
+
+
+@pytest.mark.parametrize("act", ["float16", "bfloat16"])
+@pytest.mark.parametrize("D,out,gs,counts", [
+    (256, 528, 64, [1, 0, 31, 32, 33]),          # four k-steps, a last n-tile of 16 columns
+    (768, 256, 64, [19, 20, 20, 21, 0, 20]),     # a half trip; 16.7 rows an expert: 32-row tiles
+    (1024, 512, 128, [40, 63, 64, 65, 1, 0]),    # groups of 128; 64-row tiles, a second m-tile
+    (2048, 512, 64, [96, 1, 2, 97]),             # the upper end of the range
+])
+def test_mid_gemm_is_bit_identical(D, out, gs, counts, act, monkeypatch):
+    """The mid-batch GEMM (32- and 64-row tiles) against the register-staged
+    128-row kernel, which sums in the same order: grouped products with
+    ragged, empty and shuffled experts."""
+    from nano_vllm_metal_amd import grouped_expert_linear
+
+    rng = np.random.default_rng(D + out)
+    E, n = len(counts), sum(counts)
+    w = qweights(_packed(rng, E, out, D, gs, act), act, gs, DEV)
+    x = to_act(O.round_act(rng.standard_normal((n, D)), act), act, DEV)
+    ids = torch.from_numpy(rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int32))
+    mid = grouped_expert_linear(x, w, ids.to(DEV), regime="prefill")
+    monkeypatch.setenv("NVM_GEMM_NODMA", "1")
+    ref = grouped_expert_linear(x, w, ids.to(DEV), regime="prefill")
+    assert torch.equal(mid, ref)
+
+
+@pytest.mark.parametrize("act", ["float16", "bfloat16"])
+@pytest.mark.parametrize("M,N,K,gs", [
+    (520, 1024, 528, 64),    # one block of rows a tile
+    (1500, 4096, 2048, 128),  # two
+    (1000, 768, 1024, 64),
+])
+def test_mid_gemm_dense_is_bit_identical(M, N, K, gs, act, monkeypatch):
+    """Dense products whose 128-row grid is small, as above; with SwiGLU too."""
+    from nano_vllm_metal_amd.linear import quantized_linear, quantized_swiglu
+
+    rng = np.random.default_rng(M)
+    ws = [qweights(tuple(t[0] for t in _packed(rng, 1, K, N, gs, act)), act, gs, DEV)
+          for _ in range(2)]
+    x = to_act(O.round_act(rng.standard_normal((M, N)), act), act, DEV)
+    mid = quantized_linear(x, ws[0]), quantized_swiglu(x, *ws)
+    monkeypatch.setenv("NVM_GEMM_NODMA", "1")
+    ref = quantized_linear(x, ws[0]), quantized_swiglu(x, *ws)
+    assert torch.equal(mid[0], ref[0]) and torch.equal(mid[1], ref[1])
+
+
 @pytest.mark.parametrize("act", ["float16", "bfloat16"])
 @pytest.mark.parametrize("T,H,E,k", [
     (128, 2048, 128, 8),   # whole 16-token blocks, eight hidden splits
