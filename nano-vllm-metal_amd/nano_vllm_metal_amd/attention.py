@@ -9,8 +9,6 @@ torch tensors on one GPU; there is no CPU fallback.
 
 from __future__ import annotations
 
-import ctypes
-
 import torch
 
 from . import _lib
@@ -72,16 +70,15 @@ def paged_attention(query: torch.Tensor, key_pages: torch.Tensor, value_pages: t
         raise ValueError(f"paged_attention: unsupported out_dtype {out_dtype}")
     out = torch.empty((B * Hq, L, D), dtype=out_dtype, device=dev)
     kv = _lib.KV_DTYPE_CODES[key_pages.dtype]
-    size = ctypes.c_size_t(0)
-    _lib.check(lib.nvm_paged_attention_workspace_size(B * Hq, L, D, bt.shape[1], page_size, kv,
-                                                      Hkv, Hq, ctypes.byref(size)))
-    ws = torch.empty(max(size.value, 1), dtype=torch.uint8, device=dev)
+    size = _lib.workspace_size("nvm_paged_attention_workspace_size", B * Hq, L, D, bt.shape[1],
+                               page_size, kv, Hkv, Hq)
+    ws = torch.empty(max(size, 1), dtype=torch.uint8, device=dev)
     _lib.check(lib.nvm_paged_attention(
         q.data_ptr(), B * Hq, L, D, kp.data_ptr(), vp.data_ptr(), P, page_size, kv,
         _lib.ptr(ks), _lib.ptr(vs), bt.data_ptr(), B, bt.shape[1], lens.data_ptr(),
         float(factor), int(mask == "causal"), Hkv, Hq, _lib.KV_DTYPE_CODES[out_dtype],
         out.data_ptr(), ws.data_ptr(),
-        size.value, _lib.stream_of(dev)))
+        size, _lib.stream_of(dev)))
     return out.reshape(B, Hq, L, D)
 
 

@@ -129,7 +129,7 @@ def quantized_matmul(scales: torch.Tensor, biases: torch.Tensor, group_size: int
         raise ValueError("quantized_matmul: a, scales and biases must share a dtype")
     dev = _lib.require_device(a, b, scales, biases)
     *lead, N = a.shape
-    a2 = a.reshape(-1, N).contiguous()
+    a2 = (a if len(lead) == 1 else a.reshape(-1, N)).contiguous()
     b = _u32_view_as_i32(b).contiguous()
     scales = scales.contiguous()
     biases = biases.contiguous()
@@ -143,23 +143,26 @@ def quantized_matmul(scales: torch.Tensor, biases: torch.Tensor, group_size: int
         scales.data_ptr(), biases.data_ptr(), group_size, bits, a2.data_ptr(), b.data_ptr(),
         int(bool(transpose_b)), out.data_ptr(), a2.shape[0], N, K, _lib.dtype_code(a.dtype),
         _lib.stream_of(dev)))
-    return out.reshape(*lead, K)
+    return out if len(lead) == 1 else out.reshape(*lead, K)
 
 
 def swiglu_supports(x: torch.Tensor, w_gate: QuantizedWeights, w_up: QuantizedWeights) -> bool:
     """Whether ``quantized_swiglu`` takes these operands: one shape, group
     size and dtype for both weights, and a product that ``quantized_matmul``
     does not run on its exact float64 path."""
-    K, words = w_gate.weight.shape if w_gate.weight.dim() == 2 else (0, 0)
-    N = x.shape[-1]
-    M = x.numel() // N if N else 0
-    return (w_up.weight.shape == w_gate.weight.shape and words * 8 == N
-            and w_gate.group_size == w_up.group_size and w_gate.bits == w_up.bits == 4
-            and all(t.dtype == x.dtype and t.shape == (K, N // w_gate.group_size)
-                    for w in (w_gate, w_up) for t in (w.scales, w.biases))
-            and w_gate.group_size in (64, 128) and x.dtype in _lib.DTYPE_CODES
-            and M > 0 and (K > 512 or M > 64) and K % 16 == 0 and N % w_gate.group_size == 0
-            and N <= 8192)
+    shape, gs, act, N = w_gate.weight.shape, w_gate.group_size, x.dtype, x.shape[-1]
+    if len(shape) != 2 or w_up.weight.shape != shape or w_up.group_size != gs \
+            or gs not in (64, 128) or not w_gate.bits == w_up.bits == 4:
+        return False
+    K = shape[0]
+    if shape[1] * 8 != N or not 0 < N <= 8192 or N % gs or K % 16 or act not in _lib.DTYPE_CODES:
+        return False
+    per_row = (K, N // gs)
+    for t in (w_gate.scales, w_gate.biases, w_up.scales, w_up.biases):
+        if t.dtype != act or t.shape != per_row:
+            return False
+    M = x.numel() // N
+    return M > 0 and (K > 512 or M > 64)
 
 
 def quantized_swiglu(x: torch.Tensor, w_gate: QuantizedWeights, w_up: QuantizedWeights
@@ -174,15 +177,16 @@ def quantized_swiglu(x: torch.Tensor, w_gate: QuantizedWeights, w_up: QuantizedW
                               w_up.scales, w_up.biases)
     *lead, N = x.shape
     a = x.reshape(-1, N).contiguous()
-    gw, uw = (_u32_view_as_i32(w.weight).contiguous() for w in (w_gate, w_up))
-    gsc, gbi, usc, ubi = (t.contiguous() for w in (w_gate, w_up) for t in (w.scales, w.biases))
+    gw, uw = _u32_view_as_i32(w_gate.weight).contiguous(), _u32_view_as_i32(w_up.weight).contiguous()
+    gsc, gbi = w_gate.scales.contiguous(), w_gate.biases.contiguous()
+    usc, ubi = w_up.scales.contiguous(), w_up.biases.contiguous()
     K = gw.shape[0]
     out = torch.empty((a.shape[0], K), dtype=x.dtype, device=dev)
     _lib.check(lib.nvm_quantized_swiglu(
         gsc.data_ptr(), gbi.data_ptr(), gw.data_ptr(), usc.data_ptr(), ubi.data_ptr(),
         uw.data_ptr(), w_gate.group_size, w_gate.bits, a.data_ptr(), out.data_ptr(), a.shape[0],
         N, K, _lib.dtype_code(x.dtype), _lib.stream_of(dev)))
-    return out.reshape(*lead, K)
+    return out if len(lead) == 1 else out.reshape(*lead, K)
 
 
 def quantized_linear(x: torch.Tensor, w: QuantizedWeights,

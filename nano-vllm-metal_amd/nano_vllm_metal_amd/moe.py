@@ -191,15 +191,12 @@ class Moe:
                 for w in (self.w_router, self.w_gate, self.w_up, self.w_down)]
 
     def _workspace(self, T: int, H: int, I: int, E: int, dev: torch.device) -> torch.Tensor:
-        size = ctypes.c_size_t()
-        lib = _lib.load()
-        _lib.check(lib.nvm_moe_workspace_size(T, H, I, E, self.num_experts_per_tok,
-                                              ctypes.byref(size)))
-        if self._ws is None or self._ws.numel() < size.value or self._ws.device != dev:
+        need = _lib.workspace_size("nvm_moe_workspace_size", T, H, I, E,
+                                   self.num_experts_per_tok)
+        if self._ws is None or self._ws.numel() < need or self._ws.device != dev:
             # A HIP graph captured earlier may still refer to the old buffer:
             # it stays alive with the block.  Replacements at least double
             # in size, so the retired buffers total less than the current one.
-            need = size.value
             if self._ws is not None:
                 if self._ws.device == dev:
                     need = max(need, 2 * self._ws.numel())
