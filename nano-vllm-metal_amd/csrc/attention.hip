@@ -415,6 +415,12 @@ __global__ __launch_bounds__(256) void paged_combine_kernel(const float *__restr
   const int64_t n = blockIdx.x;
   const float *ml = part_ml + n * S * 2;
   const int t = threadIdx.x;
+  // the first splits' outputs of dim t are requested before the weights are
+  // known: one round trip less for the rows of up to eight splits
+  float pre[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u)
+    pre[u] = t < D && u < S ? part_o[(n * S + u) * D + t] : 0.f;
   if (t < 64) {
     // wavefront 0: the row maximum and the weighted sum of the L_s
     float M = -INFINITY;
@@ -437,6 +443,16 @@ __global__ __launch_bounds__(256) void paged_combine_kernel(const float *__restr
     const float *po = part_o + n * S * D + d;
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     int s = 0;
+    if (d == t && S < 8) {
+#pragma unroll
+      for (int u = 0; u < 7; ++u)
+        if (u < S) acc[0] += s_w[u] * pre[u];
+      s = S;
+    } else if (d == t) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc[u] += s_w[u] * pre[u];
+      s = 8;
+    }
     for (; s + 8 <= S; s += 8) {
 #pragma unroll
       for (int u = 0; u < 8; ++u) acc[u] += s_w[s + u] * po[(int64_t)(s + u) * D];
