@@ -35,11 +35,12 @@ constexpr int MW_PITCH = 72;      // scale/bias window rows, as gemm.hip
 constexpr int MW_WAVE = 32 * MW_PITCH;
 constexpr int kARing = 4;         // k-steps of activations in registers
 
-constexpr int stage_lds(int NI) { return 2 * 32 * NI * MA_PITCH + 4 * MW_WAVE; }
+// KB: k-steps between two barriers (2 KB activation stages)
+constexpr int stage_lds(int NI, int KB) { return 2 * KB * 32 * NI * MA_PITCH + 4 * MW_WAVE; }
 template <bool DUAL>
-constexpr int mid_lds(int NI) {
+constexpr int mid_lds(int NI, int KB) {
   const int out = 32 * NI * (2 * (DUAL ? MWROWS / 2 : MWROWS) + 16);
-  return out > stage_lds(NI) ? out : stage_lds(NI);
+  return out > stage_lds(NI, KB) ? out : stage_lds(NI, KB);
 }
 
 // (nothing moves across: the rings' loads stay in the k-step that issues them)
@@ -50,7 +51,7 @@ __device__ __forceinline__ void step_fence() {
 
 // NI: 32-row blocks of routed rows per tile; kWRing: k-steps of weights in
 // registers.
-template <int DT, bool DUAL, bool AH, bool G128, int NI>
+template <int DT, bool DUAL, bool AH, bool G128, int NI, int KB>
 __global__ __launch_bounds__(256, NI == 1 ? 3 : 2) void gemm_mid_kernel(const GroupedArgs a,
                                                                        int n_tiles) {
   using A = Act<DT>;
@@ -64,7 +65,7 @@ __global__ __launch_bounds__(256, NI == 1 ? 3 : 2) void gemm_mid_kernel(const Gr
   // tile's rows are known
   int *const s_tiles = (int *)smem;
   int *const s_offs = s_tiles + kMaxExperts + 1;
-  static_assert(2 * (kMaxExperts + 1) * 4 <= stage_lds(NI), "m-tile list exceeds the staging LDS");
+  static_assert(2 * (kMaxExperts + 1) * 4 <= stage_lds(NI, KB), "m-tile list exceeds the staging LDS");
 
   hoist_args(a.act, a.act_ld, a.act_rows, a.a_map, a.a_div, a.offsets, a.w0, a.s0, a.b0, a.w1,
              a.s1, a.b1, a.R, a.K, a.E, a.out, a.o_map, a.out_ld, n_tiles);
@@ -183,7 +184,7 @@ __global__ __launch_bounds__(256, NI == 1 ? 3 : 2) void gemm_mid_kernel(const Gr
         wcur[2 * s + t2] = bload8(r, gh < GPR ? srow[s] + 8 * h : kMaskedOffset, so);
       }
   };
-  uint8_t *const w_lds = smem + 2 * MA_STAGE + wv * MW_WAVE + l32 * MW_PITCH;
+  uint8_t *const w_lds = smem + 2 * KB * MA_STAGE + wv * MW_WAVE + l32 * MW_PITCH;
   auto new_window = [&](int wi) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -256,23 +257,29 @@ __global__ __launch_bounds__(256, NI == 1 ? 3 : 2) void gemm_mid_kernel(const Gr
     }
   };
 
-  // k-step ks computes LDS buffer ks & 1; its activations' register slot
-  // (stored a step earlier) takes those of ks + 4, its weights' slot, after
-  // the pair's second step, those of kWRing k-steps on
+  // k-step ks computes LDS buffer ks % (2 KB); its activations' register slot
+  // (stored before the last barrier) takes those of ks + 4, its weights'
+  // slot, after the pair's second step, those of kWRing k-steps on
   auto k_loop = [&](auto NA) {
     auto trip = [&](int ks0, auto N) {
 #pragma unroll
       for (int j = 0; j < decltype(N)::value; ++j) {
         const int ks = ks0 + j;
-        issue_a(xa[j % kARing], ks + kARing);
-        step_fence();
+        if (j % KB == 0) {
+#pragma unroll
+          for (int d = 0; d < KB; ++d) issue_a(xa[(j + d) % kARing], ks + d + kARing);
+          step_fence();
+        }
         if (j == 0 && (!G128 || (ks0 & 8) == 0)) new_window(ks0 >> (G128 ? 4 : 3));
         take_sb(G128 ? ((ks0 & 8) + j) >> 1 : j);
-        compute(j & 1, wq[j % kWRing], NA);
+        compute(j % (2 * KB), wq[j % kWRing], NA);
         if (j & 1) issue_b(wq[(j - 1) % kWRing], wq[j % kWRing], ks - 1 + kWRing);
-        step_fence();
-        store(xa[(j + 1) % kARing], (j + 1) & 1);
-        __syncthreads();
+        if (j % KB == KB - 1) {
+          step_fence();
+#pragma unroll
+          for (int d = 1; d <= KB; ++d) store(xa[(j + d) % kARing], (j + d) % (2 * KB));
+          __syncthreads();
+        }
       }
     };
     int ks0 = 0;
@@ -345,7 +352,8 @@ __global__ __launch_bounds__(256, NI == 1 ? 3 : 2) void gemm_mid_kernel(const Gr
   if (shifted) {
     shifted_loop();
   } else {
-    store(xa[0], 0);
+#pragma unroll
+    for (int d = 0; d < KB; ++d) store(xa[d], d);
     __syncthreads();
     if (NI > 1 && mcnt > 32)
       k_loop(std::integral_constant<int, NI>{});
@@ -409,25 +417,32 @@ __global__ __launch_bounds__(256, NI == 1 ? 3 : 2) void gemm_mid_kernel(const Gr
   }
 }
 
-template <int DT, bool DUAL, bool AH, int NI>
+template <int DT, bool DUAL, bool AH, int NI, int KB>
 hipError_t launch_n(const GroupedArgs &a, int64_t pairs, hipStream_t st) {
   constexpr int cols = DUAL ? MWROWS / 2 : MWROWS;
   const int n_tiles = (a.R + cols - 1) / cols;
   const int64_t max_m_tiles = pairs / (32 * NI) + a.E;
   const unsigned grid = (unsigned)(8 * ((max_m_tiles * n_tiles + 7) / 8));
   if (a.gs == 128)
-    hipLaunchKernelGGL((gemm_mid_kernel<DT, DUAL, AH, true, NI>), dim3(grid), dim3(256),
-                       mid_lds<DUAL>(NI), st, a, n_tiles);
+    hipLaunchKernelGGL((gemm_mid_kernel<DT, DUAL, AH, true, NI, KB>), dim3(grid), dim3(256),
+                       mid_lds<DUAL>(NI, KB), st, a, n_tiles);
   else
-    hipLaunchKernelGGL((gemm_mid_kernel<DT, DUAL, AH, false, NI>), dim3(grid), dim3(256),
-                       mid_lds<DUAL>(NI), st, a, n_tiles);
+    hipLaunchKernelGGL((gemm_mid_kernel<DT, DUAL, AH, false, NI, KB>), dim3(grid), dim3(256),
+                       mid_lds<DUAL>(NI, KB), st, a, n_tiles);
   return hipGetLastError();
 }
 
+// Two k-steps a barrier where a CU holds one block (dense products: 4096 ->
+// 2048 at 1500 rows 43.5 -> 41.0 us) or three (32-row tiles: 0.5 % of a
+// layer); with two co-resident blocks, which cover each other's barriers, one
+// (700 tokens at hidden 4096: 493 against 500 us).
 template <int DT, bool DUAL, bool AH>
 hipError_t launch_t(int ni, const GroupedArgs &a, int64_t pairs, hipStream_t st) {
-  return ni == 1 ? launch_n<DT, DUAL, AH, 1>(a, pairs, st)
-                 : launch_n<DT, DUAL, AH, 2>(a, pairs, st);
+  if (ni == 1) return launch_n<DT, DUAL, AH, 1, 2>(a, pairs, st);
+  if constexpr (!AH) {
+    if (!a.offsets) return launch_n<DT, DUAL, AH, 2, 2>(a, pairs, st);
+  }
+  return launch_n<DT, DUAL, AH, 2, 1>(a, pairs, st);
 }
 
 }  // namespace
