@@ -180,32 +180,43 @@ __global__ __launch_bounds__(64 * kCW) void causal_prefill_kernel(CausalArgs a) 
   // the wavefront's columns all exist and see every key below wp0 + 1
   const bool all_cols = wp0 + PPW <= a.L;
 
-  // staging loads of tile kt into registers (rows past kend read as zeros)
+  // staging loads of tile kt into registers, through descriptors that start at
+  // the tile's first row and end with its last row below kend (rows past it
+  // read as zeros): a thread's offsets are the same for every tile, and the
+  // descriptors are scalar work.  (64-bit addresses and a branch per load took
+  // some 150 of 650 VALU instructions a wavefront and tile: 5 x 1001 tokens
+  // 148.4 us, 143 with this and the key operands read a 16-key row ahead.)
   f32x4 kreg[KI][2], vreg[VI][4];
+  const int row_b = a.Hkv * DH * 4;  // bytes between rows of one head
+  int koff[KI], voff[VI];
+#pragma unroll
+  for (int i = 0; i < KI; ++i) {
+    const int item = tid + 64 * kCW * i;
+    koff[i] = item < KN ? item / DG * row_b + 32 * (item % DG) : kMaskedOffset;
+  }
+#pragma unroll
+  for (int i = 0; i < VI; ++i) {
+    const int item = tid + 64 * kCW * i;
+    voff[i] = item < VN ? item / DG * 2 * row_b + 32 * (item % DG) : kMaskedOffset;
+  }
   auto stage_load = [&](int kt) {
+    const int64_t first = ((tok0 + kt * kKT) * a.Hkv + kvh) * DH;
+    const int rows = min(kKT, kend - kt * kKT);
+    const uint32_t bytes = (uint32_t)((rows - 1) * row_b + DH * 4);
+    const rsrc_t kr = make_rsrc(a.k + first, bytes), vr = make_rsrc(a.v + first, bytes);
 #pragma unroll
-    for (int i = 0; i < KI; ++i) {
-      const int item = tid + 64 * kCW * i;
-      const int key = item / DG, dg = item - key * DG;
-      const int j = kt * kKT + key;
-      const bool ok = item < KN && j < kend;
-      const float *kp = a.k + ((tok0 + (ok ? j : 0)) * a.Hkv + kvh) * DH + 8 * dg;
-      kreg[i][0] = ok ? *(const f32x4 *)kp : f32x4{0.f, 0.f, 0.f, 0.f};
-      kreg[i][1] = ok ? *(const f32x4 *)(kp + 4) : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int i = 0; i < KI; ++i)
 #pragma unroll
-    for (int i = 0; i < VI; ++i) {
-      const int item = tid + 64 * kCW * i;
-      const int kp2 = item / DG, dg = item - kp2 * DG;
+      for (int x = 0; x < 2; ++x)
+        kreg[i][x] = __builtin_bit_cast(f32x4, bload16(kr, koff[i] + 16 * x, 0));
 #pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        const int j = kt * kKT + 2 * kp2 + r;
-        const bool ok = item < VN && j < kend;
-        const float *vp = a.v + ((tok0 + (ok ? j : 0)) * a.Hkv + kvh) * DH + 8 * dg;
-        vreg[i][2 * r] = ok ? *(const f32x4 *)vp : f32x4{0.f, 0.f, 0.f, 0.f};
-        vreg[i][2 * r + 1] = ok ? *(const f32x4 *)(vp + 4) : f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-    }
+    for (int i = 0; i < VI; ++i)
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+          vreg[i][2 * r + x] =
+              __builtin_bit_cast(f32x4, bload16(vr, voff[i] + r * row_b + 16 * x, 0));
   };
   auto stage_store = [&](int buf) {
 #pragma unroll
@@ -253,16 +264,25 @@ __global__ __launch_bounds__(64 * kCW) void causal_prefill_kernel(CausalArgs a) 
     // S^T: keys 16u + c16 as the A operand (dims 32kk + 8G .. +7), each key
     // operand read once for the column tiles
     f32x4 acc[CT][4];
+    u32x4 kop[2][NC];
+    auto load_k = [&](int u) {
+#pragma unroll
+      for (int kk = 0; kk < NC; ++kk)
+        kop[u & 1][kk] = *(const u32x4 *)&s_k[buf][16 * u + c16][32 * kk + 8 * G];
+    };
+    load_k(0);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
+      if (u < 3) load_k(u + 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) acc[ct][u] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int kk = 0; kk < NC; ++kk) {
-        const u32x4 kop = *(const u32x4 *)&s_k[buf][16 * u + c16][32 * kk + 8 * G];
+      for (int kk = 0; kk < NC; ++kk)
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) acc[ct][u] = A::mfma16(kop, qop[ct][kk], acc[ct][u]);
-      }
+        for (int ct = 0; ct < CT; ++ct)
+          acc[ct][u] = A::mfma16(kop[u & 1][kk], qop[ct][kk], acc[ct][u]);
+      __builtin_amdgcn_sched_barrier(0);
     }
     // Causal mask (key j <= position, j < L), base-2 scores, online softmax.
     // Interior tiles (every key of the tile visible to every column of the
