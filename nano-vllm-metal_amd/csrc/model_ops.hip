@@ -192,8 +192,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(QkvArgs a) {
   const int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (item >= a.T * NH) return;
   const int lane = threadIdx.x & 63;
-  // (32 bits hold every item: a 64-bit division is a long software sequence)
-  const int64_t t = (uint32_t)item / (uint32_t)NH;
+  // (a 64-bit division is a long software sequence)
+  const int64_t t = a.T * NH <= 0xFFFFFFFFll ? (uint32_t)item / (uint32_t)NH : item / NH;
   const int head = (int)(item - t * NH);
   const int D2 = a.D / 2, half = a.D / 2, Q = a.D / 4;  // pairs per head, half dims, lane offset
   const bool on = lane < D2;
