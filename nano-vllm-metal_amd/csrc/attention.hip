@@ -546,7 +546,7 @@ AttnPlan attn_plan(int64_t N, int64_t L, int64_t D, int64_t max_pages, int64_t p
                    int kv_dtype, int Hkv, int Hq) {
   AttnPlan p{false, 0, 1, 1, 0};
   p.decode = L == 1 && kv_dtype != NVM_KV_F32 && (D == 64 || D == 128);
-  if (!p.decode) return p;
+  if (!p.decode || N == 0) return p;  // (an empty batch has no blocks to share out)
   const int R = Hq / Hkv;
   p.RP = R <= 8 ? 8 : 16;
   p.HG = (R + p.RP - 1) / p.RP;

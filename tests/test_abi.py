@@ -290,6 +290,17 @@ def test_paged_attention_workspace_size():
     assert sz.value == 0
 
 
+@pytest.mark.parametrize("kv_dtype", [0, 1, 2, 3])
+def test_paged_attention_workspace_size_of_an_empty_batch(kv_dtype):
+    """No requests need no workspace, whatever the page dtype (the split plan
+    divides by the number of blocks, which is zero then)."""
+    _, lib = _lib()
+    sz = ctypes.c_size_t(1)
+    assert lib.nvm_paged_attention_workspace_size(0, 1, 128, 80, 16, kv_dtype, 4, 32,
+                                                  ctypes.byref(sz)) == 0
+    assert sz.value == 0
+
+
 @pytest.mark.parametrize("call,code,msg", [
     (lambda lib: lib.nvm_residual_rms_norm(1, 1, 1, 4, 2047, 1e-6, 1, 1, 1, None), -1, "bad shape"),
     (lambda lib: lib.nvm_residual_rms_norm(1, 1, 1, 4, 16384, 1e-6, 1, 1, 1, None), -2, "at most"),
