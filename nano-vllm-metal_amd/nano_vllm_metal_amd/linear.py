@@ -148,12 +148,14 @@ def quantized_matmul(scales: torch.Tensor, biases: torch.Tensor, group_size: int
 
 def swiglu_supports(x: torch.Tensor, w_gate: QuantizedWeights, w_up: QuantizedWeights) -> bool:
     """Whether ``quantized_swiglu`` takes these operands: one shape, group
-    size and dtype for both weights, and a product that ``quantized_matmul``
-    does not run on its exact float64 path."""
+    size and dtype for both weights, 32-bit words, and a product that
+    ``quantized_matmul`` does not run on its exact float64 path."""
     shape, gs, act, N = w_gate.weight.shape, w_gate.group_size, x.dtype, x.shape[-1]
     if len(shape) != 2 or w_up.weight.shape != shape or w_up.group_size != gs \
             or gs not in (64, 128) or not w_gate.bits == w_up.bits == 4:
         return False
+    if not w_gate.weight.element_size() == w_up.weight.element_size() == 4:
+        return False  # (the shape below counts 32-bit words)
     K = shape[0]
     if shape[1] * 8 != N or not 0 < N <= 8192 or N % gs or K % 16 or act not in _lib.DTYPE_CODES:
         return False

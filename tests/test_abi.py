@@ -301,6 +301,25 @@ def test_paged_attention_workspace_size_of_an_empty_batch(kv_dtype):
     assert sz.value == 0
 
 
+@pytest.mark.parametrize("dtype,takes", [
+    (torch.int32, True), (torch.uint32, True), (torch.int64, False), (torch.int16, False),
+    (torch.uint8, False),
+])
+def test_swiglu_takes_32bit_words_only(dtype, takes):
+    """Weights of another element size than the packed words' are refused by
+    the separate products (their int32 view has another shape), so the fused
+    gate/up product does not take them either: it would read past their end."""
+    from nano_vllm_metal_amd import QuantizedWeights
+    from nano_vllm_metal_amd.linear import swiglu_supports
+
+    x = torch.zeros(4, 2048, dtype=torch.bfloat16)
+    s = torch.zeros(1024, 32, dtype=torch.bfloat16)
+    words = QuantizedWeights(s, s, 64, 4, torch.zeros(1024, 256, dtype=torch.int32))
+    other = QuantizedWeights(s, s, 64, 4, torch.zeros(1024, 256, dtype=dtype))
+    assert swiglu_supports(x, other, words) is takes
+    assert swiglu_supports(x, words, other) is takes
+
+
 @pytest.mark.parametrize("call,code,msg", [
     (lambda lib: lib.nvm_residual_rms_norm(1, 1, 1, 4, 2047, 1e-6, 1, 1, 1, None), -1, "bad shape"),
     (lambda lib: lib.nvm_residual_rms_norm(1, 1, 1, 4, 16384, 1e-6, 1, 1, 1, None), -2, "at most"),
