@@ -131,10 +131,15 @@ def stream_of(device: torch.device) -> int:
         torch.cuda.current_device() if index is None else index)
 
 
-@functools.lru_cache(maxsize=512)
 def workspace_size(name: str, *shape: int) -> int:
     """Workspace bytes of entry point `name` (its ``nvm_*_workspace_size``),
-    which depend on the shape arguments alone."""
+    which depend on the shape arguments and on the current device: the
+    library's splits follow its number of compute units."""
+    return _workspace_size(torch.cuda.current_device(), name, *shape)
+
+
+@functools.lru_cache(maxsize=512)
+def _workspace_size(device: int, name: str, *shape: int) -> int:
     size = ctypes.c_size_t()
     check(getattr(load(), name)(*shape, ctypes.byref(size)))
     return size.value

@@ -301,6 +301,32 @@ def test_paged_attention_workspace_size_of_an_empty_batch(kv_dtype):
     assert sz.value == 0
 
 
+def test_workspace_sizes_are_kept_per_device(monkeypatch):
+    """A size asked for on one device is not reused on another: the splits
+    behind it follow the device's compute units."""
+    L, _ = _lib()
+    current = 0
+    asked = []
+
+    class Library:
+        @staticmethod
+        def nvm_moe_workspace_size(T, size):
+            asked.append((current, T))
+            size._obj.value = 1000 * (current + 1) + T
+            return 0
+
+    monkeypatch.setattr(L, "load", lambda: Library)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current)
+    L._workspace_size.cache_clear()
+    try:
+        sizes = []
+        for current in (0, 1, 0, 1):
+            sizes.append(L.workspace_size("nvm_moe_workspace_size", 7))
+    finally:
+        L._workspace_size.cache_clear()
+    assert sizes == [1007, 2007, 1007, 2007] and asked == [(0, 7), (1, 7)]
+
+
 @pytest.mark.parametrize("dtype,takes", [
     (torch.int32, True), (torch.uint32, True), (torch.int64, False), (torch.int16, False),
     (torch.uint8, False),
