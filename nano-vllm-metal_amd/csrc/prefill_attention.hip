@@ -118,7 +118,9 @@ __device__ __forceinline__ int vt_col(int r, int kp) {
   return pc ^ vt_swz((r >> 4) & 7);
 }
 
-template <int DT, int DH, int R, int CT>
+// WIDE: the rows of a tile span more than a descriptor's 32-bit offsets reach
+// (launch_causal_r); they are loaded through 64-bit addresses.
+template <int DT, int DH, int R, int CT, bool WIDE>
 __global__ __launch_bounds__(64 * kCW) void causal_prefill_kernel(CausalArgs a) {
   using A = Act<DT>;
   constexpr int NC = DH / 32;       // 32-dim steps of a score MFMA
@@ -192,16 +194,45 @@ __global__ __launch_bounds__(64 * kCW) void causal_prefill_kernel(CausalArgs a) 
 #pragma unroll
   for (int i = 0; i < KI; ++i) {
     const int item = tid + 64 * kCW * i;
-    koff[i] = item < KN ? item / DG * row_b + 32 * (item % DG) : kMaskedOffset;
+    // (keys past the request's end: L rows are all whose offsets fit 32 bits)
+    koff[i] =
+        item < KN && item / DG < a.L ? item / DG * row_b + 32 * (item % DG) : kMaskedOffset;
   }
 #pragma unroll
   for (int i = 0; i < VI; ++i) {
     const int item = tid + 64 * kCW * i;
-    voff[i] = item < VN ? item / DG * 2 * row_b + 32 * (item % DG) : kMaskedOffset;
+    voff[i] = item < VN && item / DG * 2 < a.L ? item / DG * 2 * row_b + 32 * (item % DG)
+                                               : kMaskedOffset;
   }
   auto stage_load = [&](int kt) {
     const int64_t first = ((tok0 + kt * kKT) * a.Hkv + kvh) * DH;
     const int rows = min(kKT, kend - kt * kKT);
+    if constexpr (WIDE) {
+#pragma unroll
+      for (int i = 0; i < KI; ++i) {
+        const int item = tid + 64 * kCW * i;
+        const bool ok = item < KN && item / DG < rows;
+        const float *kp =
+            a.k + first + (ok ? (int64_t)(item / DG) * a.Hkv * DH + 8 * (item % DG) : 0);
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+          kreg[i][x] = ok ? *(const f32x4 *)(kp + 4 * x) : f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int i = 0; i < VI; ++i) {
+        const int item = tid + 64 * kCW * i;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+          const int key = 2 * (item / DG) + r;
+          const bool ok = item < VN && key < rows;
+          const float *vp = a.v + first + (ok ? (int64_t)key * a.Hkv * DH + 8 * (item % DG) : 0);
+#pragma unroll
+          for (int x = 0; x < 2; ++x)
+            vreg[i][2 * r + x] = ok ? *(const f32x4 *)(vp + 4 * x) : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+      return;
+    }
     const uint32_t bytes = (uint32_t)((rows - 1) * row_b + DH * 4);
     const rsrc_t kr = make_rsrc(a.k + first, bytes), vr = make_rsrc(a.v + first, bytes);
 #pragma unroll
@@ -400,12 +431,19 @@ hipError_t launch_causal_r(const CausalArgs &a0, int R, hipStream_t st) {
                        a);
     return hipGetLastError();
   };
+  // (tensors of fewer than 2^31 elements: only one or two query heads a kv
+  // head leave room for 64 rows of 2 GiB)
+  if ((int64_t)std::min(kKT, a.L) * a.Hkv * DH * 4 > kMaskedOffset) {
+    if (R == 1) return go(causal_prefill_kernel<DT, DH, 1, kCT, true>, kCW * kCT * 16);
+    if (R == 2) return go(causal_prefill_kernel<DT, DH, 2, kCT, true>, kCW * kCT * 8);
+    return hipErrorInvalidValue;
+  }
   switch (R) {
-    case 1: return go(causal_prefill_kernel<DT, DH, 1, kCT>, kCW * kCT * 16);
-    case 2: return go(causal_prefill_kernel<DT, DH, 2, kCT>, kCW * kCT * 8);
-    case 4: return go(causal_prefill_kernel<DT, DH, 4, kCT>, kCW * kCT * 4);
-    case 8: return go(causal_prefill_kernel<DT, DH, 8, kCT>, kCW * kCT * 2);
-    case 16: return go(causal_prefill_kernel<DT, DH, 16, kCT>, kCW * kCT);
+    case 1: return go(causal_prefill_kernel<DT, DH, 1, kCT, false>, kCW * kCT * 16);
+    case 2: return go(causal_prefill_kernel<DT, DH, 2, kCT, false>, kCW * kCT * 8);
+    case 4: return go(causal_prefill_kernel<DT, DH, 4, kCT, false>, kCW * kCT * 4);
+    case 8: return go(causal_prefill_kernel<DT, DH, 8, kCT, false>, kCW * kCT * 2);
+    case 16: return go(causal_prefill_kernel<DT, DH, 16, kCT, false>, kCW * kCT);
     default: return hipErrorInvalidValue;
   }
 }

@@ -340,6 +340,29 @@ def test_causal_attention_30b_heads_8x1024():
                                        err_msg=f"b={b} h={h}")
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,act", [
+    (70_000, 70_000, 128, torch.bfloat16),   # 64 rows span 2.3 GB
+    (262_200, 131_100, 64, torch.float16),
+])
+def test_causal_attention_rows_beyond_32bit_offsets(Hq, Hkv, D, act):
+    """A 64-key tile whose rows lie further apart than 32-bit offsets reach
+    (65 tokens: a second tile of one key), against the oracle on heads at
+    both ends and in the middle."""
+    from nano_vllm_metal_amd.attention import causal_attention
+
+    L, r, scale = 65, Hq // Hkv, D ** -0.5
+    g = torch.Generator(device=DEV).manual_seed(3)
+    q, k, v = (torch.randn(1, L, h, D, device=DEV, generator=g).to(act).float()
+               for h in (Hq, Hkv, Hkv))
+    out = causal_attention(q, k, v, scale, act)
+    for h in (0, 1, Hq // 2 - 1, Hq - 2, Hq - 1):
+        kvh = h // r
+        ref = _causal_ref(q[:, :, h:h + 1].cpu(), k[:, :, kvh:kvh + 1].cpu(),
+                          v[:, :, kvh:kvh + 1].cpu(), 0, 0, scale)
+        np.testing.assert_allclose(out[0, :, h].cpu().numpy(), ref, rtol=1e-4, atol=2e-5,
+                                   err_msg=f"h={h}")
+
+
 def test_causal_attention_rejects_unsupported_shapes():
     from nano_vllm_metal_amd.attention import causal_attention
 
