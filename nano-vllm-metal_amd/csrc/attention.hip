@@ -405,7 +405,12 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(PagedArgs a) {
 // Splits of a row: out = sum_s 2^(M_s - M) O_s / sum_s 2^(M_s - M) L_s.
 // One block per row: the splits' (M_s, L_s) are read in parallel into LDS,
 // then thread d sums its dim over the splits with the loads of eight splits
-// in flight at a time.
+// in flight at a time.  FEW (at most eight splits, D at most the block's
+// threads): the outputs are requested before the weights are known, one
+// round trip less (7 splits of one request at 32/4 heads: 4.4 us a launch
+// without, 3.1 with; 8: 3.2 / 3.1).  More splits keep the plain loop: with
+// the first eight requested ahead 9 to 64 of them took 0.2 to 0.8 us longer.
+template <bool FEW>
 __global__ __launch_bounds__(256) void paged_combine_kernel(const float *__restrict__ part_o,
                                                             const float *__restrict__ part_ml,
                                                             int S, int D, void *out,
@@ -415,12 +420,12 @@ __global__ __launch_bounds__(256) void paged_combine_kernel(const float *__restr
   const int64_t n = blockIdx.x;
   const float *ml = part_ml + n * S * 2;
   const int t = threadIdx.x;
-  // the first splits' outputs of dim t are requested before the weights are
-  // known: one round trip less for the rows of up to eight splits
   float pre[8];
+  if constexpr (FEW) {
 #pragma unroll
-  for (int u = 0; u < 8; ++u)
-    pre[u] = t < D && u < S ? part_o[(n * S + u) * D + t] : 0.f;
+    for (int u = 0; u < 8; ++u)
+      pre[u] = t < D && u < S ? part_o[(n * S + u) * D + t] : 0.f;
+  }
   if (t < 64) {
     // wavefront 0: the row maximum and the weighted sum of the L_s
     float M = -INFINITY;
@@ -442,22 +447,24 @@ __global__ __launch_bounds__(256) void paged_combine_kernel(const float *__restr
   for (int d = t; d < D; d += 256) {
     const float *po = part_o + n * S * D + d;
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    int s = 0;
-    if (d == t && S < 8) {
+    if constexpr (FEW) {
+      // (in the order of the loop below)
+      if (S < 8) {
 #pragma unroll
-      for (int u = 0; u < 7; ++u)
-        if (u < S) acc[0] += s_w[u] * pre[u];
-      s = S;
-    } else if (d == t) {
+        for (int u = 0; u < 7; ++u)
+          if (u < S) acc[0] += s_w[u] * pre[u];
+      } else {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) acc[u] += s_w[u] * pre[u];
-      s = 8;
+        for (int u = 0; u < 8; ++u) acc[u] += s_w[u] * pre[u];
+      }
+    } else {
+      int s = 0;
+      for (; s + 8 <= S; s += 8) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc[u] += s_w[s + u] * po[(int64_t)(s + u) * D];
+      }
+      for (; s < S; ++s) acc[0] += s_w[s] * po[(int64_t)s * D];
     }
-    for (; s + 8 <= S; s += 8) {
-#pragma unroll
-      for (int u = 0; u < 8; ++u) acc[u] += s_w[s + u] * po[(int64_t)(s + u) * D];
-    }
-    for (; s < S; ++s) acc[0] += s_w[s] * po[(int64_t)s * D];
     const float o = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
     store_out(out, out_dt, n * D + d, o * s_inv);
   }
@@ -718,8 +725,10 @@ int nvm_paged_attention(const float *q, int64_t N, int64_t L, int64_t D, const v
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(NVM_ERR_HIP, "paged_attention: %s", hipGetErrorString(e));
     if (plan.S > 1) {
-      hipLaunchKernelGGL(paged_combine_kernel, dim3((unsigned)N), dim3(256), 0, st, a.part_o,
-                         a.part_ml, plan.S, (int)D, out, out_dtype);
+      // (decode rows have at most 128 dims)
+      hipLaunchKernelGGL(plan.S <= 8 ? paged_combine_kernel<true> : paged_combine_kernel<false>,
+                         dim3((unsigned)N), dim3(256), 0, st, a.part_o, a.part_ml, plan.S, (int)D,
+                         out, out_dtype);
       e = hipGetLastError();
       if (e != hipSuccess)
         return set_error(NVM_ERR_HIP, "paged_attention combine: %s", hipGetErrorString(e));

@@ -178,6 +178,14 @@ def test_int8_multi_query_causal():
     _run(109, 2, 8, 4, 64, 16, [33, 100], L=4, causal=True, int8=True)
 
 
+@pytest.mark.parametrize("ctx", [100, 448, 512, 576, 1024])
+@pytest.mark.parametrize("D,dtype", [(128, "bfloat16"), (64, "float16")])
+def test_split_merge(ctx, D, dtype):
+    """One request at one split a 64-position tile: 2, 7, 8, 9 and 16 splits
+    (the merge takes up to eight another way)."""
+    _run(130 + ctx, 1, 8, 2, D, 16, [ctx], dtype=dtype, causal=True)
+
+
 @pytest.mark.parametrize("Hq,Hkv,D,ps,lens", [
     (8, 8, 64, 4, [1, 63, 64, 65, 0]),         # one head per kv head, edges of a 64-position tile
     (10, 2, 128, 24, [511, 513, 700]),         # five per kv head, edges of a block's eight tiles
