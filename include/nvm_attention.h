@@ -52,7 +52,8 @@ enum nvm_kv_dtype { NVM_KV_F16 = 0, NVM_KV_BF16 = 1, NVM_KV_F32 = 2, NVM_KV_I8 =
  * decode kernel (the query heads of a kv head share every page read); L > 1
  * with f16/bf16 pages and those D runs a matrix-core kernel over the pages;
  * other shapes run a one-wavefront-per-row kernel (so do int8 pages or a
- * query not aligned to 16 bytes).  Each page tensor must be below 2 GiB.
+ * query not aligned to 16 bytes, and int8 tables of a few positions a request
+ * for many requests).  Each page tensor must be below 2 GiB.
  * Workspace: nvm_paged_attention_workspace_size (zero bytes when no split is
  * needed; workspace may then be NULL).  Int8 pages are also accepted without
  * a workspace: the context is then not split.

@@ -39,9 +39,9 @@
 //     multiplies its float32 score and its value scale the probability before
 //     the split into three parts, so every product stays exact and both sums
 //     float32.
-// Other shapes (L > 1 on f32 or int8 pages, f32 decode, other head dims) run
-// one wavefront per query row over the context, with the reference's formula
-// per element.
+// Other shapes (L > 1 on f32 or int8 pages, f32 decode, other head dims, int8
+// decode of many short contexts) run one wavefront per query row over the
+// context, with the reference's formula per element.
 #include <math.h>
 
 #include <algorithm>
@@ -173,8 +173,9 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(PagedArgs a) {
   const int p1 = min(p0 + a.span, ctx);
 
   // B operand of the score MFMAs (query head c16, dims 32k + 8G .. +7, or in
-  // the order of the 16-code key loads), the same for every wavefront: built once into LDS, read back per tile (it
-  // would hold 12 * NC VGPRs for the whole loop)
+  // the order of the 16-code key loads), the same for every wavefront: built
+  // once into LDS, read back per tile (it would hold 12 * NC VGPRs for the
+  // whole loop)
   if (wv == 0) {
     const bool ok = c16 < nh;
     const float *qp = a.q + (n0 + (ok ? c16 : 0)) * DH;
@@ -549,6 +550,22 @@ struct AttnPlan {
   int RP, HG, S, span;
 };
 
+// Int8 decode over short contexts, on the row kernel?  A row's wavefront takes
+// about 1 us a position, more from 18 wavefronts a CU on; a block of the
+// decode kernel some 8 us at any length up to its first eight tiles, a CU
+// running one at a time (two at D = 64).  By table capacity `cap`, the most a
+// context can hold.  Row / decode kernel, us a call: 32/4 heads of 128, 256
+// requests of up to 16 positions 25.6 / 34.2, of 32 44.7 / 34.9; 16/16 heads
+// of 128, 64 requests of up to 16: 16.2 / 31.7, 32: 29.4 / 32.1, 48: 42.5 /
+// 32.3; 512 requests of up to 64: 116 / 270, 160: 326 / 293; 8/8 heads of 64,
+// 512 requests of up to 48: 46.6 / 48.8, 64: 69.4 / 51.4.  (32/1 heads, whose
+// blocks take 16 rows and 11 us, lose up to 2 us at 8 positions.)
+bool int8_rows(int64_t rows, int64_t blocks, int64_t D, int64_t cap) {
+  const double cu = cu_count();
+  return (double)cap * std::max(1.0, (double)rows / (18 * cu)) <=
+         8.0 * std::max(1.0, (double)blocks / (D == 64 ? 2 * cu : cu));
+}
+
 AttnPlan attn_plan(int64_t N, int64_t L, int64_t D, int64_t max_pages, int64_t page_size,
                    int kv_dtype, int Hkv, int Hq) {
   AttnPlan p{false, 0, 1, 1, 0};
@@ -559,6 +576,8 @@ AttnPlan attn_plan(int64_t N, int64_t L, int64_t D, int64_t max_pages, int64_t p
   p.HG = (R + p.RP - 1) / p.RP;
   const int64_t tiles = (max_pages * page_size + kTile - 1) / kTile;
   const int64_t base = N / Hq * Hkv * p.HG;
+  if (kv_dtype == NVM_KV_I8 && int8_rows(N, base, D, max_pages * page_size))
+    return AttnPlan{false, 0, 1, 1, 0};
   const int64_t s0 = std::max<int64_t>(1, (kTargetBlocks + base - 1) / base);
   int64_t tps = std::max<int64_t>(1, (tiles + s0 - 1) / s0);
   tps = std::max<int64_t>(tps, (tiles + kMaxSplits - 1) / kMaxSplits);

@@ -200,6 +200,19 @@ def test_int8_decode_matrix_cores(Hq, Hkv, D, ps, lens):
          causal=Hq % 3 == 0)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,D,ps,cap", [
+    (64, 16, 16, 128, 16, 32),    # four blocks a CU: the row kernel
+    (64, 16, 16, 128, 16, 48),    # and the decode kernel
+    (80, 32, 4, 64, 8, 8),        # one block a CU: below and
+    (80, 32, 4, 64, 1, 9),        # above eight positions
+])
+def test_int8_decode_of_many_short_contexts(B, Hq, Hkv, D, ps, cap):
+    """Both sides of the line between the row and the decode kernel."""
+    lens = np.random.default_rng(cap).integers(0, cap + 1, B)
+    lens[0] = cap
+    _run(150 + cap, B, Hq, Hkv, D, ps, lens, int8=True, holes=1)
+
+
 def test_int8_decode_without_workspace_or_alignment():
     """Int8 decode calls accepted before the split kernel took them: no
     workspace (one split per row), codes at an odd address (the row kernel).
