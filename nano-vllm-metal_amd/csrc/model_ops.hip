@@ -97,7 +97,7 @@ void launch_norm(const void *h, const void *r, const void *w, int64_t T, int H2,
 // MoE combine + residual add + RMSNorm, one block per token: the token's k
 // expert outputs summed in slot order exactly as the combine kernel does
 // (y = rnd(sum_j rnd(down_j * score_j))), then h_out = rnd(h + y) and
-// x_out = rnd(rms_norm(h_out) * w).  Eight pairs' loads are in flight at once
+// x_out = rnd(rms_norm(h_out) * w).  Several pairs' loads are in flight at once
 // (KK: the top-k as a compile-time count, every pair's loads at once, the
 // float32 halves included; the arithmetic and its order are the same).
 constexpr int kCombChunks = 4;  // 8-value chunks per thread: H <= 256 * 4 * 8
@@ -127,8 +127,11 @@ __global__ __launch_bounds__(kNormThreads) void moe_combine_residual_norm_kernel
     const u32x4 hh = ldg16(h + t * H + 8 * c);
     wq[q] = ldg16(w + 8 * c);
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    // pairs whose loads are in flight together (KK: all of them)
-    constexpr int NB = KK ? KK : SPLIT ? 4 : 8;
+    // pairs whose loads are in flight together (KK: all of them).  Four in
+    // fp16: eight pairs' conversions took 252 registers and 32 accumulation
+    // registers, one wavefront a SIMD (4096 tokens of 2048, top-6: 83 us a
+    // launch; 31 with four, 108 registers)
+    constexpr int NB = KK ? KK : SPLIT || DT == DT_F16 ? 4 : 8;
     for (int j0 = 0; j0 < k; j0 += NB) {
       float dv[NB][8];
       uint32_t sv[NB];

@@ -98,7 +98,8 @@ def test_qk_norm_rope_store(Hq, Hkv, D, dt, wide):
 
 
 @pytest.mark.parametrize("T,dt,k", [(32, torch.bfloat16, 4), (300, torch.float16, 4),
-                                    (32, torch.bfloat16, 8), (64, torch.float16, 8)])
+                                    (32, torch.bfloat16, 8), (64, torch.float16, 8),
+                                    (300, torch.float16, 5), (300, torch.bfloat16, 9)])
 def test_moe_combine_residual_norm(T, dt, k):
     """nvm_moe_forward_residual_norm: h_out is bit-identical to h + Moe(x)
     (the combine's arithmetic, then one rounding), x_out the norm of it;
