@@ -497,18 +497,31 @@ bool route_i8_fin_supports(int64_t T, int64_t H, int64_t E, int gs, int k) {
 }
 
 // The one-launch routing runs T / 16 blocks, each a chain of a quarter of the
-// hidden columns' k-steps and the finalise: 30 us at any T up to 4096 (H
-// 2048), 58 us at H 4096.  Over hidden splits the partial logits of 150
-// tokens take 8 us and the finalise 6.  The layer's time with one launch /
-// two (bf16): H 2048, 150 tokens 170.7 / 155.2 us, 512 183.8 / 169.9, 1000
-// 215.5 / 219.2, 2048 312.4 / 305.6, 3000 376.0 / 379.3; H 4096, 150 tokens
-// 484.5 / 451.5, 700 556.5 / 536.6, 1000 625.6 / 614.1.
+// hidden columns' k-steps and the finalise.  Over hidden splits the partial
+// logits and the finalise of 16 tokens a block are two short launches.
+// Routing and dispatch, one launch / two (us, bf16, 128 experts): H 2048, 128
+// tokens 33.0 / 18.0, 512 34.3 / 22.0, 1000 35.6 / 27.7, 1900 37.0 / 31.0, 2500
+// 37.6 / 40.2; H 4096, 512 tokens 55.4 / 25.0, 1900 57.5 / 41.5, 2500 58.4 /
+// 58.1; H 1024, 128 tokens 23.1 / 17.2, 1900 26.4 / 26.0, 2500 25.5 / 30.0.
+// Reductions of few k-steps gain nothing from a split: H 512 with 32 experts
+// 15.6 / 16.5 at 512 tokens, H 768 with 64 17.2 / 20.0, H 512 with 128 21.1 /
+// 19.2 at 600 and 20.2 / 22.6 at 1900.
+//
+// Splits: what two blocks a CU hold at once, since a grid of three or four
+// ran in two rounds (H 2048, 1000 tokens: eight splits 35.9, four 27.7; H
+// 1024, 1900 tokens: four 31.9, two 26.0); up to three where half the splits
+// would leave a wavefront more than four k-steps (H 4096, 1150 tokens: four
+// 36.1, two 39.1; 1900 tokens, 3.7 blocks: four 46.3, two 41.5).
 constexpr int64_t kRouteSplitTokens = 2048;
 int route_i8_split(int64_t T, int64_t H, int64_t E) {
-  if (T > kRouteSplitTokens) return 0;
-  const int s = route_i8_splits(T, H, E);
-  if (s < route_workspace_splits(T, H, E)) return s;
-  return s >= 2 && (H / 64 + s / 2 - 1) / (s / 2) + 1 <= kSbGroups ? s / 2 : 0;
+  const int64_t n_ec = (E + 16 * kI8Tiles - 1) / (16 * kI8Tiles), KS = H / 64;
+  if (T > kRouteSplitTokens || KS * n_ec < (T > 1024 ? 24 : 16)) return 0;
+  int s = route_i8_splits(T, H, E);
+  const int64_t blocks = (T + 15) / 16 * n_ec;
+  while (s > 1 && blocks * s > (KS > 8 * s ? 3 : 2) * cu_count()) s /= 2;
+  // (the finalise's histograms lie behind the partials: one split of room)
+  if (s == route_workspace_splits(T, H, E)) s /= 2;
+  return s >= 1 && (KS + s - 1) / s + 1 <= kSbGroups ? s : 0;
 }
 
 hipError_t launch_route_i8_fin(int dtype, const void *x, int64_t T, int64_t H, const uint32_t *wr,

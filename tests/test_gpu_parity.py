@@ -275,8 +275,12 @@ def test_mid_gemm_dense_is_bit_identical(M, N, K, gs, act, monkeypatch):
     (128, 2048, 128, 8),   # whole 16-token blocks, eight hidden splits
     (129, 2048, 40, 3),    # a last block of one token
     (333, 4096, 128, 8),   # half the splits (room for the histograms)
-    (2048, 1024, 64, 16),  # the largest batch, fewer splits
-    (2049, 1024, 64, 16),  # beyond it: one launch
+    (2048, 1024, 64, 16),  # few k-steps of a large batch: one launch
+    (2048, 2048, 64, 16),  # the largest batch, two splits
+    (2049, 2048, 64, 16),  # beyond it: one launch
+    (1000, 2048, 128, 8),  # splits that two blocks a CU hold
+    (1200, 4096, 128, 8),  # three blocks a CU
+    (2049, 1024, 64, 16),
     (200, 192, 128, 8),    # one split only: one launch
 ])
 def test_split_prefill_routing(T, H, E, k, act):
