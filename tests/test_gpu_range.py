@@ -12,7 +12,8 @@ cases send through the forward, at the 30B-A3B shape in the prefill regime:
 * rows whose values span more than 40 binades (2^-40 .. 2^20 around N(0,1));
 
 for the int8 router's batches (T >= 128: it writes the fp16 copy of x) and
-for smaller batches (the separate conversion launch).  Router ids and scores
+for smaller batches (the separate conversion launch), on each of the three
+GEMMs that read the copies.  Router ids and scores
 must equal the oracle's bit for bit; the outputs must meet the block
 tolerance row by row (relative to each row's largest reference value) and
 the reference suite's elementwise allclose.
@@ -44,8 +45,15 @@ def _wide_x(seed, T, H, act):
     return O.round_act(x, act)
 
 
-@pytest.mark.parametrize("T", [512, 96])
-def test_prefill_operands_beyond_fp16_range(T):
+@pytest.mark.parametrize("T,nodma", [
+    (512, "0"),    # 32 rows an expert: the mid-batch GEMM
+    (96, "0"),     # the separate conversion launch
+    (1000, "0"),   # more than 48 rows an expert: the direct-to-LDS GEMM
+    (1000, "1"),   # the register-staged 128-row GEMM
+    (96, "1"),
+])
+def test_prefill_operands_beyond_fp16_range(T, nodma, monkeypatch):
+    monkeypatch.setenv("NVM_GEMM_NODMA", nodma)
     act, H, E, I, gs, k = "bfloat16", 2048, 128, 768, 64, 8
     _, w = O.make_packed_inputs(500 + T, 1, H, E, I, act, gs)
     x = _wide_x(501 + T, T, H, act)
