@@ -174,10 +174,11 @@ def test_quantized_matmul_matches_oracle(M, N, K, act, gs):
 
 
 # Dense projections (more than 512 outputs, or more than 64 rows) run on the
-# expert GEMV (N <= 4096; up to 32 rows, or up to 512 while the GEMM grid
-# would be smaller than the chip) or the GEMM, accumulating in float32 like
-# quantized_matmul.metal:25-44.  The
-# GEMV's sums equal the unrounded dequantised products; the GEMM rounds each
+# few-row kernel (N a multiple of 128, few blocks), the expert GEMV (N <=
+# 4096; up to 32 rows, or up to 512 while the GEMM grid would be smaller than
+# the chip) or the GEMM, accumulating in float32 like
+# quantized_matmul.metal:25-44.  The few-row kernel's and the GEMV's sums
+# equal the unrounded dequantised products ("gemv"); the GEMM rounds each
 # dequantised weight to fp16 (single rounding of q*s + b) before its fp16
 # MFMA, 2^-12 relative, below the output rounding of either activation dtype.
 # Both are held to the tolerance against the exactly rounded oracle (outputs
@@ -191,7 +192,8 @@ def test_quantized_matmul_matches_oracle(M, N, K, act, gs):
     (3, 1024, 528, "bfloat16", 64, "gemv"),      # output tile past the last row
     (17, 2048, 768, "bfloat16", 64, "gemv"),     # two chunks, the second of one row
     (300, 1024, 4096, "float16", 64, "gemv"),    # 19 chunks (GEMM grid of 48 blocks)
-    (5, 6144, 1024, "bfloat16", 128, "gemm"),    # N the GEMV does not slice
+    (5, 6144, 1024, "bfloat16", 128, "gemv"),    # N the GEMV does not slice: few-row kernel
+    (400, 6144, 1024, "bfloat16", 128, "gemm"),  # and beyond its blocks the GEMM
     (600, 1024, 1024, "float16", 64, "gemm"),    # beyond 512 rows, ragged last tile
     (700, 2048, 768, "bfloat16", 64, "gemm"),
     (65, 2048, 512, "bfloat16", 64, "gemv"),     # narrow output beyond 64 rows
@@ -327,12 +329,30 @@ def test_few_row_dense_products(M, N, K, act, gs):
 
 
 @pytest.mark.parametrize("act", ["float16", "bfloat16"])
-@pytest.mark.parametrize("M,gs", [(1, 64), (16, 128), (33, 64), (700, 64)])
+@pytest.mark.parametrize("gs", [64, 128])
+@pytest.mark.parametrize("N,K", [(2048, 3072), (4096, 2048)])
+def test_few_row_products_equal_the_unit_list(N, K, gs, act):
+    """Reductions of 2048 and 4096 are summed in one order by the few-row
+    kernel (16 rows) and the unit-list GEMV (64 rows): a row's product, and
+    its gate/up pair with SwiGLU, do not depend on which of them ran."""
+    from nano_vllm_metal_amd.linear import quantized_linear, quantized_swiglu
+
+    rng = np.random.default_rng(N + gs)
+    ws = [qweights(tuple(t[0] for t in _packed(rng, 1, K, N, gs, act)), act, gs, DEV)
+          for _ in range(2)]
+    x = to_act(O.round_act(rng.standard_normal((64, N)), act), act, DEV)
+    assert torch.equal(quantized_linear(x[:16], ws[0]), quantized_linear(x, ws[0])[:16])
+    assert torch.equal(quantized_swiglu(x[:16], *ws), quantized_swiglu(x, *ws)[:16])
+
+
+@pytest.mark.parametrize("act", ["float16", "bfloat16"])
+@pytest.mark.parametrize("M,gs", [(1, 64), (16, 128), (33, 64), (40, 128), (400, 64),
+                                  (700, 64)])
 def test_swiglu_product_matches_separate_products(M, gs, act):
-    """quantized_swiglu (few-row, unit-list GEMV and GEMM) against silu and
-    multiply on the two separate products, each op rounded to act: bit
-    identical where both run the same kernel's sums, and in all cases within
-    the block tolerance."""
+    """quantized_swiglu (few-row kernel, unit-list GEMV at 33 and 40 rows,
+    gemv3 at 400, GEMM at 700) against silu and multiply on the two separate
+    products, each op rounded to act: bit identical where both run the same
+    kernel's sums, and in all cases within the block tolerance."""
     from nano_vllm_metal_amd.linear import quantized_linear, quantized_swiglu
     from nano_vllm_metal_amd.qwen3 import silu
 
