@@ -18,7 +18,9 @@ decode attention, the full 48-layer model through LLM.generate (32 x 1024-token
 prompts, 256 greedy tokens: end-to-end decode tokens/s), and the CPU baseline (the C restatement of the reference algorithm in oracle/,
 timed on a bounded sample).
 
-Prints one JSON line on stdout; progress goes to stderr.
+Prints one JSON line on stdout; progress goes to stderr.  The line carries
+the headline and each workload's main figures; ``--record FILE`` writes every
+timing.
 """
 
 from __future__ import annotations
@@ -1115,6 +1117,50 @@ def rocprof_summary(root: Path, write_traffic: bool) -> str:
     return text
 
 
+# The figures of each workload that the printed line carries (what a reader of
+# one line compares); the whole record goes to the file of --record.
+LINE_FIELDS = {
+    "decode": ("layer_us", "layer_us_median", "tokens_per_s", "hbm_gbs"),
+    "prefill": ("layer_us", "tokens_per_s", "layer_tflops", "in_layer_gateup_tflops",
+                "in_layer_down_tflops"),
+    "moe_235b": ("layer_us", "tokens_per_s", "hbm_gbs", "layer_tflops"),
+    "dense": ("us",),
+    "attention": ("us", "gbs", "tflops"),
+    "e2e": ("decode_tokens_per_s", "decode_step_ms", "prefill_tokens_per_s",
+            "generated_tokens_per_s"),
+    "cpu_baseline": ("value", "unit", "cores", "kind", "sample", "tokens_per_s",
+                     "routing_matches_gpu"),
+    "roofline": ("kernel", "bound", "achieved", "peak", "unit", "frac", "avg_launch_us",
+                 "algorithmic_bytes_per_launch", "traffic", "rocprof_avg_us",
+                 "frac_from_rocprof"),
+    "prefill_roofline": ("kernel", "bound", "achieved", "peak", "unit", "frac", "avg_launch_us",
+                         "layer_frac", "traffic", "rocprof_avg_us", "frac_from_rocprof"),
+}
+
+
+def line_of(record: dict) -> str:
+    """The JSON line of a record: every field of the headline, the chosen
+    figures of the rest, numbers to six significant digits.  (The whole
+    record is some 15 KB, longer than what a log's tail keeps of a line.)"""
+
+    def digits(v):
+        if isinstance(v, float):
+            return float(f"{v:.6g}")
+        if isinstance(v, dict):
+            return {k: digits(x) for k, x in v.items()}
+        return v
+
+    def pick(v, fields):
+        kept = {k: pick(x, fields) if isinstance(x, dict) else x for k, x in v.items()
+                if isinstance(x, dict) or k in fields or k == "error"}
+        return {k: x for k, x in kept.items() if x != {}}
+
+    headline = ("value", "ms_per_step")  # as measured
+    return json.dumps({k: v if k in headline else digits(pick(v, LINE_FIELDS[k]))
+                       if k in LINE_FIELDS and isinstance(v, dict) else digits(v)
+                       for k, v in record.items()})
+
+
 def main():
     ap = argparse.ArgumentParser(description=__doc__.split("\n")[0])
     ap.add_argument("--gpus", type=int, default=1)
@@ -1139,6 +1185,8 @@ def main():
     ap.add_argument("--e2e", action="store_true",
                     help="measure only the full 48-layer model through LLM.generate "
                          "(32 x 1024-token prompts, 256 greedy tokens)")
+    ap.add_argument("--record", metavar="FILE",
+                    help="write the whole record (every timing, with notes) to FILE as JSON")
     ap.add_argument("--rocprof-summary", metavar="DIR",
                     help="summarise rocprofv3 CSV output under DIR and exit (no GPU)")
     ap.add_argument("--write-traffic", action="store_true",
@@ -1361,7 +1409,9 @@ def main():
         log(f"[bench] CPU baseline: {cb['value']:.0f} tokens/s on {cb['cores']} threads, "
             f"{cb['single_thread']['tokens_per_s']:.0f} tokens/s on 1 thread "
             f"({cb['host']['cpu_model']})")
-    print(json.dumps(out), flush=True)
+    if args.record:
+        Path(args.record).write_text(json.dumps(out, indent=1) + "\n")
+    print(line_of(out), flush=True)
 
 
 if __name__ == "__main__":
