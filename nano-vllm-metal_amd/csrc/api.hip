@@ -410,14 +410,19 @@ const char *nvm_last_error(void) { return g_err.c_str(); }
 constexpr int64_t kExactOutMax = 512;
 constexpr int64_t kExactRowsMax = 64;
 
-// Kernel of a dense product of M rows over a reduction of N into K outputs.
-// The GEMV streams the weights once per 16- or 32-row chunk; the GEMM once,
-// but a block runs all N/64 k-steps in sequence, so a grid of fewer blocks
-// than CUs leaves the GEMM latency-bound.  The few-row kernel wherever it
-// applies; else the unit-list GEMV up to two chunks, and up to 32 chunks
-// while the GEMM grid would not fill the chip.
-static bool dense_decode(int64_t M, int64_t N, int64_t K) {
-  if (nvm::gemv_dense_supports(M, (int)N, (int)K)) return true;
+// Kernel of a dense product of M rows over a reduction of N into K outputs
+// (dual: the gate/up pair).  The few-row kernel wherever it applies; else the
+// unit-list GEMV, which streams the weights once per 16- or 32-row chunk, up
+// to two chunks, and up to 32 chunks while the 128-row GEMM's grid would not
+// fill the chip.  From some 150 rows on the GEMM's 32-row tiles (gemm_mid.hip)
+// are the faster side of that line (us, GEMV / GEMM: 2048 -> 5120 64 rows 12.3
+// / 18.4, 128 16.8 / 18.4, 200 25.6 / 19.3, 512 44.5 / 25.2; 4096 -> 2048 256
+// rows 23.4 / 31.1, 512 37.0 / 31.7; pair 2048 -> 6144 64 rows 17.2 / 19.8,
+// 128 26.4 / 21.1, 512 64.5 / 41.4), but they round each weight to fp16: the
+// error against 64 bits of an fp16 product is 2.07e-4 on the GEMV and 2.79e-4
+// there (bf16: 1.66e-3 on both), so batches that ran on exact weights stay.
+static bool dense_decode(bool dual, int64_t M, int64_t N, int64_t K) {
+  if (nvm::gemv_dense_supports(dual, M, (int)N, (int)K)) return true;
   const int64_t gemm_blocks = (M + nvm::kGemmBM - 1) / nvm::kGemmBM * ((K + 255) / 256);
   return nvm::gemv_supports((int)N) &&
          (M <= 32 || (M <= 512 && gemm_blocks < nvm::cu_count()));
@@ -472,7 +477,7 @@ int nvm_quantized_matmul(const void *scales, const void *biases, int group_size,
                 "split the product", (long long)(M * N * 2), (long long)(K * (N / 2)));
   if (dense_on_products(M, N, K)) {
     nvm::GroupedArgs g = dense_args(scales, biases, group_size, a, b, out, M, N, K);
-    return run_products(dtype, dense_decode(M, N, K), false, g, M, (hipStream_t)stream);
+    return run_products(dtype, dense_decode(false, M, N, K), false, g, M, (hipStream_t)stream);
   }
   NVM_TRY_HIP(nvm::launch_route_partial(dtype, a, M, N, b, scales, biases, K, group_size, true,
                                         nullptr, out, nullptr, (hipStream_t)stream));
@@ -501,7 +506,7 @@ int nvm_quantized_swiglu(const void *gate_scales, const void *gate_biases, const
   g.w1 = up;
   g.s1 = (const uint16_t *)up_scales;
   g.b1 = (const uint16_t *)up_biases;
-  return run_products(dtype, dense_decode(M, N, K), true, g, M, (hipStream_t)stream);
+  return run_products(dtype, dense_decode(true, M, N, K), true, g, M, (hipStream_t)stream);
 }
 
 int nvm_route_workspace_size(int64_t T, int64_t H, int64_t E, size_t *bytes) {

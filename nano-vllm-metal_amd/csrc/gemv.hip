@@ -623,7 +623,8 @@ hipError_t launch_gemv(int dtype, bool dual, const GroupedArgs &a, hipStream_t s
   // loads in flight: q_proj (2048 -> 4096) at one row takes 5.7 us here and
   // 9.4 us on gemv3.
   // Dense products of few rows have a kernel of their own.
-  if (!a.offsets && a.E == 1 && !a.a_map && !a.o_map && gemv_dense_supports(a.act_rows, a.K, a.R))
+  if (!a.offsets && a.E == 1 && !a.a_map && !a.o_map &&
+      gemv_dense_supports(dual, a.act_rows, a.K, a.R))
     return launch_gemv_dense(dtype, dual, a, st);
   GemvShape s;
   const bool old_ok = gemv_shape(a.K, a.R, s);

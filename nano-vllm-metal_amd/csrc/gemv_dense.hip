@@ -238,23 +238,39 @@ hipError_t launch_t(bool dual, const GroupedArgs &a, hipStream_t st) {
 
 }  // namespace
 
-// The line is drawn on the number of blocks, each of which reads its weights
-// and 16 rows of x anew.  Against the unit-list GEMV, us a call (bf16, groups
-// of 64, weights rotated past the last-level cache's reach of a call): 2048
-// -> 5120, 320 blocks a chunk: 16 rows 6.7 / 7.6, 32 rows 8.9 / 9.0, 48 rows
-// 11.0 / 12.9, 64 rows 13.3 / 12.7; 2048 -> 16384, 1024 a chunk: 1 row 10.8
-// / 9.3; so up to 2.5 blocks a CU.  4096 -> 2048, 128 a chunk: 1 row 6.8 /
-// 8.3, 32 rows 7.6 / 10.5, 48 rows 12.9 / 15.7, 64 rows 13.1 / 12.7; 4096 ->
-// 4096: 16 rows 7.7 / 10.7, 32 rows 13.1 / 12.7; up to 1.5 blocks a CU (the
-// longer ring leaves registers for fewer).  Where that GEMV does not hold
-// the reduction (K 5120, 6144, 8192) the alternative is the GEMM, whose few
-// blocks run every k-step in sequence (gemm_mid.hip): 6144 -> 2048 128 rows
-// 30.5 / 47, 160 rows 37.6 / 47, 200 rows 51.5 / 47; up to 5 blocks a CU
-// there.
-bool gemv_dense_supports(int64_t M, int K, int R) {
+// The line is drawn on the number of blocks a CU, each of which reads its
+// weights and 16 rows of x anew, against the unit-list GEMV (us a call, that
+// GEMV / this kernel, bf16, groups of 64, weights rotated past the last-level
+// cache; fp16 and groups of 128 alike).  That GEMV runs 1, 2, 4 or 8 chunks
+// of 16 rows well and other counts unevenly.
+//  * K below 2048, 2.5 blocks: 1536 -> 10240, 1 row 8.0 / 7.4; 1024 -> 5120,
+//    17 rows 7.6 / 5.7.
+//  * K 2048, two blocks: 2048 -> 8192, 1 row 7.1 / 7.1, 16 rows 7.9 / 7.4; 2048
+//    -> 4096, 32 rows 7.3 / 6.7; beyond it 2048 -> 10240, 1 row 7.8 / 9.2, and
+//    2048 -> 5120, 17 rows 8.7 / 9.0.  2.5 blocks for other chunk counts: 2048
+//    -> 3072, 33 rows 9.3 / 8.5; 2048 -> 1024, 145 rows 10.5 / 8.5.
+//  * K up to 3072, 1.5 blocks: 2560 -> 6144, 1 row 9.3 / 9.4, 16 rows 11.0 /
+//    10.0; 2560 -> 9216 11.2 / 13.1.
+//  * K up to 4096, one block (the longer ring leaves registers for one): 4096
+//    -> 4096, 1 row 8.8 / 7.8, 4096 -> 2048, 32 rows 10.2 / 7.4; beyond it 4096
+//    -> 5120, 1 row 11.1 / 13.3, 3072 -> 6144 8.5 / 10.8.  1.5 blocks for other
+//    chunk counts: 4096 -> 2048, 33 rows 15.3 / 12.5; 3072 -> 1024, 81 rows
+//    11.8 / 9.9.
+// The gate/up pair has the same lines: 2048 -> 6144, 1 row 9.6 / 10.1, 16 rows
+// 10.6 / 10.3, 17 rows (3 blocks) 12.1 / 13.4; 2048 -> 10240 12.0 / 13.5; 4096
+// -> 4096 16.3 / 11.3, 4096 -> 6144 19.5 / 20.6.
+// Where that GEMV does not hold the reduction (K 5120, 6144, 8192) the
+// alternative is the GEMM, whose few blocks run every k-step in sequence
+// (gemm_mid.hip): 6144 -> 2048, 128 rows 46.6 / 31.1, 160 rows 46.5 / 38.1, 200
+// rows 47 / 51.5; 5120 -> 20480, 16 rows 46.1 / 42.0: five blocks there, four
+// for the pair (5120 -> 2048, 128 rows 42.6 / 44.3, fp16 41.1 / 37.0).
+bool gemv_dense_supports(bool dual, int64_t M, int K, int R) {
   if (M < 1 || M > 4096 || K % 128 || K > 8192 || R % 16) return false;
-  const int64_t blocks = (M + 15) / 16 * (R / 16), cu = cu_count();
-  return 2 * blocks <= (K <= 2048 ? 5 : 3) * cu || (!gemv_supports(K) && blocks <= 5 * cu);
+  const int64_t chunks = (M + 15) / 16, blocks = chunks * (R / 16), cu = cu_count();
+  if (!gemv_supports(K)) return blocks <= (dual ? 4 : 5) * cu;
+  const bool pow2 = (chunks & (chunks - 1)) == 0;
+  if (K <= 2048) return 2 * blocks <= (K == 2048 && pow2 ? 4 : 5) * cu;
+  return 2 * blocks <= (K >= 3072 && pow2 ? 2 : 3) * cu;
 }
 
 hipError_t launch_gemv_dense(int dtype, bool dual, const GroupedArgs &a, hipStream_t st) {

@@ -189,7 +189,7 @@ hipError_t launch_gemv3(int dtype, bool dual, const GroupedArgs &a, hipStream_t 
 // Dense products of few rows (one expert, no maps; gemv_dense.hip): K a
 // multiple of 128 up to 8192, R of 16, either group size, and a grid of
 // (R / 16) x ceil(M / 16) blocks small enough for it.
-bool gemv_dense_supports(int64_t M, int K, int R);
+bool gemv_dense_supports(bool dual, int64_t M, int K, int R);
 hipError_t launch_gemv_dense(int dtype, bool dual, const GroupedArgs &a, hipStream_t st);
 constexpr int kGemmBM = 128;   // prefill tile rows (routed pairs)
 constexpr int kGemmBN = 128;   // prefill tile columns per weight matrix
