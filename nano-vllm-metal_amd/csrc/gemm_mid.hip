@@ -34,6 +34,7 @@ constexpr int MA_PITCH = 144;     // bytes per staged activation row (128 + 16)
 constexpr int MW_PITCH = 72;      // scale/bias window rows, as gemm.hip
 constexpr int MW_WAVE = 32 * MW_PITCH;
 constexpr int kARing = 4;         // k-steps of activations in registers
+constexpr int kWRing = 4;         // k-steps of weights
 
 // KB: k-steps between two barriers (2 KB activation stages)
 constexpr int stage_lds(int NI, int KB) { return 2 * KB * 32 * NI * MA_PITCH + 4 * MW_WAVE; }
@@ -49,15 +50,13 @@ __device__ __forceinline__ void step_fence() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// NI: 32-row blocks of routed rows per tile; kWRing: k-steps of weights in
-// registers.
+// NI: 32-row blocks of routed rows per tile.
 template <int DT, bool DUAL, bool AH, bool G128, int NI, int KB>
 __global__ __launch_bounds__(256, NI == 1 ? 3 : 2) void gemm_mid_kernel(const GroupedArgs a,
                                                                        int n_tiles) {
   using A = Act<DT>;
   constexpr int MBM = 32 * NI;  // routed rows per tile
   constexpr int MA_STAGE = MBM * MA_PITCH;
-  constexpr int kWRing = NI == 1 ? 4 : 4;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   __shared__ int s_arow[MBM];
   __shared__ int s_orow[MBM];
@@ -333,9 +332,6 @@ __global__ __launch_bounds__(256, NI == 1 ? 3 : 2) void gemm_mid_kernel(const Gr
   issue_b(wq[2], wq[3], 2);
   issue_a(xa[3], 3);
   step_fence();
-#pragma unroll
-  for (int p = 4; p < kWRing; p += 2) issue_b(wq[p % kWRing], wq[(p + 1) % kWRing], p);
-  step_fence();
   // fp16 copies stored with group shifts (as gemm.hip)
   bool shifted = false;
   if constexpr (AH && DT == DT_BF16) {
@@ -456,7 +452,12 @@ hipError_t launch_t(int ni, const GroupedArgs &a, int64_t pairs, hipStream_t st)
 // goes in rounds of one block a CU: 4096 -> 2048 (fp16, groups of 128) at 600
 // rows 33 / 42 / 67, 1000 rows (256, 128, 64 blocks) 35 / 43 / 67, 1500 rows
 // (376, 192, 96) 54 / 44 / 68, 2500 rows (632, 320, 160) - / 66 / 69; 2048 ->
-// 5120 at 1500 rows (-, 480, 240) - / 42.4 / 41.5.
+// 5120 at 1500 rows (-, 480, 240) - / 42.4 / 41.5.  A second round of
+// up to a quarter of the CUs pays with groups of 128, with groups of 64 up to
+// a reduction of 4096: two blocks / 128-row kernels, groups of 128, 6144 ->
+// 2048 at 2100 rows (bf16) 93.6 / 97.3, 8192 -> 4096 at 1250 (fp16) 129 / 133;
+// groups of 64 (bf16), 4096 -> 2048 at 2500 69.3 / 69.7, 5120 -> 5120 at 800
+// 88.3 / 85.5, 8192 -> 4096 at 1250 136 / 130.
 // NVM_GEMM_NODMA=1 takes the register-staged 128-row kernel instead.
 int gemm_mid_blocks(bool dual, const GroupedArgs &a, int64_t pairs) {
   const char *v = getenv("NVM_GEMM_NODMA");
@@ -465,7 +466,8 @@ int gemm_mid_blocks(bool dual, const GroupedArgs &a, int64_t pairs) {
   const int cols = dual ? MWROWS / 2 : MWROWS;
   const int64_t nt = (a.R + cols - 1) / cols, cu = cu_count();
   if ((pairs + 31) / 32 * nt <= cu) return 1;
-  return 4 * ((pairs + 63) / 64 * nt) <= 5 * cu ? 2 : 0;
+  const int quarters = a.gs == 64 && a.K > 4096 ? 4 : 5;
+  return 4 * ((pairs + 63) / 64 * nt) <= quarters * cu ? 2 : 0;
 }
 
 hipError_t launch_gemm_mid(int dtype, bool dual, int blocks, const GroupedArgs &a, int64_t pairs,
