@@ -84,15 +84,6 @@ __device__ __forceinline__ void store_out(void *out, int dt, int64_t i, float v)
     ((uint16_t *)out)[i] = Act<DT_F16>::from_f32(v);
 }
 
-// Hand-over of LDS data between the lanes of one wavefront: its LDS
-// operations execute in program order, so only the compiler must not move
-// loads or stores across this point.
-__device__ __forceinline__ void wave_lds_sync() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_wave_barrier();
-  asm volatile("" ::: "memory");
-}
-
 // q = p0 + p1 + p2 in the page dtype, for four pairs of values.
 template <int DT>
 __device__ __forceinline__ void split3(const float (&x)[8], u32x4 &p0, u32x4 &p1, u32x4 &p2) {

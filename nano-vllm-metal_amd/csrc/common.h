@@ -175,6 +175,15 @@ __device__ __forceinline__ uint32_t perm_b32(uint32_t hi, uint32_t lo, uint32_t 
   return __builtin_amdgcn_perm(hi, lo, sel);
 }
 
+// Hand-over of LDS data between the lanes of one wavefront: its LDS
+// operations execute in program order, so only the compiler must not move
+// loads or stores across this point.
+__device__ __forceinline__ void wave_lds_sync() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // Words (w0, w1, w2, w3) of a 16-byte load in lane group G hold codes
 // 32G + 8j.. of a 128-code group pair.  Exchanging the lower half-wave's
 // words 2-3 with the upper half-wave's words 0-1 leaves every lane with words

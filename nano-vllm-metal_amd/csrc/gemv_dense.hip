@@ -34,14 +34,6 @@ namespace nvm {
 
 namespace {
 
-// LDS handed between the lanes of one wavefront: its LDS operations execute
-// in program order, so only the compiler must not move them across this point.
-__device__ __forceinline__ void wave_lds_order() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_wave_barrier();
-  asm volatile("" ::: "memory");
-}
-
 // RING: pairs in flight per wavefront, and pairs between two applications of
 // the bias terms.
 template <int DT, bool DUAL, int NW, int RING, bool G128>
@@ -115,13 +107,13 @@ __global__ __launch_bounds__(64 * NW) void gemv_dense_kernel(const GroupedArgs a
     uint8_t *const xs = s_x[wv];
 #pragma unroll
     for (int j = 0; j < 4; ++j) *(u32x4 *)(xs + (4 * j + G) * XP + 16 * col) = q.x[j];
-    wave_lds_order();
+    wave_lds_sync();
     u32x4 xa[4];
 #pragma unroll
     for (int st = 0; st < 4; ++st)
       xa[st] = *(const u32x4 *)(xs + col * XP + 64 * (G & 1) + 32 * (G >> 1) + 128 * (st >> 1) +
                                 16 * (st & 1));
-    wave_lds_order();
+    wave_lds_sync();
     float ps[2];  // the two groups' sums of x over row `col`, in every lane of it
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
