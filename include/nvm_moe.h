@@ -69,7 +69,10 @@ const char *nvm_last_error(void);
  * accumulating in float32 as the reference's kernels do
  * (quantized_matmul.metal:25-44, :100-110), when N is a multiple of 64 up to
  * 8192 and K a multiple of 16; other shapes take the float64 path (exact,
- * but bound by the float64 matrix cores: slow for large products).  Operands
+ * but bound by the float64 matrix cores: slow for large products).  Batches
+ * of few rows multiply the exact dequantised weights, larger ones weights
+ * rounded to fp16, so a row's last bits may depend on the number of rows it
+ * comes with.  Operands
  * of more than 2 GiB (a or b) are rejected with NVM_ERR_UNSUPPORTED.
  * Needs no workspace.
  */

@@ -429,7 +429,7 @@ hipError_t launch_n(const GroupedArgs &a, int64_t pairs, hipStream_t st) {
 }
 
 // Two k-steps a barrier where a CU holds one block (dense products: 4096 ->
-// 2048 at 1500 rows 43.5 -> 41.0 us) or three (32-row tiles: 0.5 % of a
+// 2048 at 1500 rows 42.8 -> 41.4 us) or three (32-row tiles: 0.5 % of a
 // layer); with two co-resident blocks, which cover each other's barriers, one
 // (700 tokens at hidden 4096: 493 against 500 us).
 template <int DT, bool DUAL, bool AH>
@@ -447,17 +447,21 @@ hipError_t launch_t(int ni, const GroupedArgs &a, int64_t pairs, hipStream_t st)
 // one / two blocks a tile / the 128-row kernels (bf16, us): 150 tokens (9 rows
 // an expert) 126 / 132 / 159, 256 (16) 130 / 135 / 163, 384 (24) 149 / 142 /
 // 161, 700 (44) 191 / 172 / 178, 1000 (62) - / 211 / 202; hidden 4096: 700
-// tokens 655 / 489 / 523, 1000 - / 617 / 584.
+// tokens 655 / 489 / 523, 1000 - / 617 / 584.  Skewed routing (the first
+// experts at 10 to 16 times the mean) leaves the line where it is: the layer
+// against the 128-row design, 150 tokens 136 / 184, 512 170 / 218, 767 198 /
+// 225; hidden 4096, 700 tokens 560 / 610.
 // Dense products: by the grid.  A block runs the whole reduction, so the time
-// goes in rounds of one block a CU: 4096 -> 2048 (fp16, groups of 128) at 600
-// rows 33 / 42 / 67, 1000 rows (256, 128, 64 blocks) 35 / 43 / 67, 1500 rows
-// (376, 192, 96) 54 / 44 / 68, 2500 rows (632, 320, 160) - / 66 / 69; 2048 ->
-// 5120 at 1500 rows (-, 480, 240) - / 42.4 / 41.5.  A second round of
-// up to a quarter of the CUs pays with groups of 128, with groups of 64 up to
-// a reduction of 4096: two blocks / 128-row kernels, groups of 128, 6144 ->
-// 2048 at 2100 rows (bf16) 93.6 / 97.3, 8192 -> 4096 at 1250 (fp16) 129 / 133;
-// groups of 64 (bf16), 4096 -> 2048 at 2500 69.3 / 69.7, 5120 -> 5120 at 800
-// 88.3 / 85.5, 8192 -> 4096 at 1250 136 / 130.
+// goes in rounds of one block a CU (fp16, groups of 128, weights rotated past
+// the caches, one / two blocks a tile / 128-row kernels, in brackets the
+// blocks): 4096 -> 2048 at 600 rows 32 / 39 / 67, 1000 rows (256, 128, 64) 36 /
+// 40 / 67, 1500 rows (376, 192, 96) 50 / 41 / 68, 2500 rows (632, 320, 160) 74 /
+// 66 / 68; 2048 -> 5120 at 1500 rows (940, 480, 240) 58 / 47 / 44.  A second
+// round of up to a quarter of the CUs pays with groups of 128, with groups of
+// 64 up to a reduction of 4096: two blocks / 128-row kernels, groups of 128,
+// 6144 -> 2048 at 2100 rows (bf16) 93.6 / 97.3, 8192 -> 4096 at 1250 (fp16)
+// 129 / 133; groups of 64 (bf16), 4096 -> 2048 at 2500 69.3 / 69.7, 5120 ->
+// 5120 at 800 88.3 / 85.5, 8192 -> 4096 at 1250 136 / 130.
 // NVM_GEMM_NODMA=1 takes the register-staged 128-row kernel instead.
 int gemm_mid_blocks(bool dual, const GroupedArgs &a, int64_t pairs) {
   const char *v = getenv("NVM_GEMM_NODMA");

@@ -215,10 +215,11 @@ hipError_t launch_n(const GroupedArgs &a, hipStream_t st) {
 
 // Reductions that the unit-list GEMV splits into eight slices (K 2048, 4096)
 // are split alike, two or four pairs a wavefront, and sum in its order: a
-// row's result is the same bit for bit from either kernel, whatever the
-// number of rows.  (4096 -> 2048 at 16 rows: 7.2 us; sixteen wavefronts of
-// two pairs took 6.7, in another order.)  Longer ones take sixteen wavefronts, the gate/up
-// pair eight (its partial sums fill twice the LDS).
+// row's result is the same bit for bit from either kernel, for the row counts
+// that either of them takes (the GEMM beyond them rounds the weights to fp16).
+// (4096 -> 2048 at 16 rows: 7.2 us; sixteen wavefronts of two pairs took 6.7,
+// in another order.)  Longer ones take sixteen wavefronts, the gate/up pair
+// eight (its partial sums fill twice the LDS).
 template <int DT>
 hipError_t launch_t(bool dual, const GroupedArgs &a, hipStream_t st) {
   if (dual)
