@@ -31,7 +31,8 @@ __device__ __forceinline__ uint32_t round_pair(float a, float b) {
 // and of the weights is issued before the first is used (past the row's end
 // through masked offsets): with a load and its use behind a bound check per
 // pair, a row of 2048 was four dependent round trips and the weights a fifth
-// behind the barrier: 8 rows 6.2 us, 4.8 this way.
+// behind the barrier: 8 rows 3.7 us among other launches, 2.4 this way (6.2 and
+// 4.8 timed alone by the profiler).
 template <int DT, int NP>
 __global__ __launch_bounds__(kNormThreads) void residual_rms_norm_kernel(
     const uint32_t *h, const uint32_t *r, const uint32_t *w, int H2, float eps, uint32_t *h_out,
